@@ -214,6 +214,9 @@ int dn_launch_sphere_edits(const DNeditParams& p, uint32_t numTiles, hipStream_t
 int dn_launch_edit_scatter(uint2* words, const uint32_t* tiles, const uint2* in, uint32_t n, hipStream_t stream);
 int dn_launch_edit_gather(const uint2* words, const uint32_t* tiles, uint2* out, uint32_t n, hipStream_t stream);
 
+// Whether DN_init has succeeded in this process.
+bool dn_initialised();
+
 // Fills the lighting-pass parameters of `vol` for a frame (engine.cpp).
 struct DNvolume;
 bool prepare_lighting(DNvolume* vol, int numDiffuseSamples, int maxDiffuseSamples, float time, DNlightParams& p,

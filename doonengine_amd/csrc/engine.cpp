@@ -845,6 +845,8 @@ uint32_t pop_eviction(DNgpuVolume* g, EvictionQueue& q, int k)
 // ===========================================================================
 // INITIALIZATION (voxel.c:119-295)
 
+namespace { std::atomic<bool> g_initialised{false}; }
+
 extern "C" bool DN_init(void)
 {
     int n = 0;
@@ -854,11 +856,11 @@ extern "C" bool DN_init(void)
         return false;
     }
     build_lut();
-    // every device's address of the allocation-free prediction's scratch array
-    if(!dn_noalloc_init())
-        dn_msg(DN_MESSAGE_GPU_MEMORY, DN_MESSAGE_ERROR, "allocation-free prediction: scratch address lookup failed");
+    g_initialised = true;
     return true;
 }
+
+bool dn_initialised() { return g_initialised; }
 
 extern "C" void DN_quit(void) {}
 

@@ -15,17 +15,39 @@ enum {
     RC_OFF_W0 = 0, RC_OFF_W1 = 3072, RC_OFF_W2 = 7168, RC_OFF_W3 = 11264, RC_NPARAM = 12288
 };
 
-// Index in the transposed weight layout (each of W0 64x48, W1 and W2 64x64,
-// W3 16x64 transposed in place, same offsets) of weight i of the row-major one.
-__host__ __device__ inline uint32_t rc_transposed_index(uint32_t i)
+// The bf16 copies of the weights are kept in the order in which the matrix
+// instructions take them, so a lane's A operand is one contiguous piece of LDS
+// (16 bytes for v_mfma_f32_16x16x32_bf16, 8 for v_mfma_f32_16x16x16_bf16) and
+// a wave's 64 pieces are consecutive: a conflict-free read. Position, within a
+// matrix of `cols` columns (16, 48 or 64), of element (row, col): 16-row blocks,
+// in each its 32-column blocks, then the 16-column block that is left over. In a
+// block, lane 16 q + r (r = row mod 16) holds the columns 4 q + 0..3 of the
+// block's one or two 16-column halves.
+__host__ __device__ inline uint32_t rc_fragment_index(uint32_t cols, uint32_t row, uint32_t col)
 {
-    uint32_t off, rows, cols;
+    const uint32_t c = col & 31u, lane = 16u * ((c & 15u) >> 2) + (row & 15u), j = c & 3u;
+    const uint32_t block = (row >> 4) * 16u * cols + (col >> 5) * 512u;
+    return (col >> 5) < (cols >> 5) ? block + lane * 8u + (c >> 4) * 4u + j : block + lane * 4u + j;
+}
+
+// Matrix that weight i belongs to: its offset, rows and columns.
+__host__ __device__ inline void rc_weight_matrix(uint32_t i, uint32_t& off, uint32_t& rows, uint32_t& cols)
+{
     if(i < RC_OFF_W1) { off = RC_OFF_W0; rows = 64; cols = 48; }
     else if(i < RC_OFF_W2) { off = RC_OFF_W1; rows = 64; cols = 64; }
     else if(i < RC_OFF_W3) { off = RC_OFF_W2; rows = 64; cols = 64; }
     else { off = RC_OFF_W3; rows = 16; cols = 64; }
-    const uint32_t j = i - off;
-    return off + (j % cols) * rows + j / cols;
+}
+
+// Positions of weight i of the row-major layout in the fragment order of its
+// matrix (forward) and of the matrix's transpose (backward).
+__host__ __device__ inline void rc_fragment_positions(uint32_t i, uint32_t& forward, uint32_t& transposed)
+{
+    uint32_t off, rows, cols;
+    rc_weight_matrix(i, off, rows, cols);
+    const uint32_t r = (i - off) / cols, c = (i - off) % cols;
+    forward = off + rc_fragment_index(cols, r, c);
+    transposed = off + rc_fragment_index(rows, c, r);
 }
 
 struct DNrcNet {
@@ -38,8 +60,8 @@ struct DNrcNet {
     float* tabGrad;
     float* tabM;
     float* tabV;
-    uint16_t* w16;                 // [RC_NPARAM] bf16
-    uint16_t* wT16;                // w16 in the transposed layout (rc_transposed_index), for backward
+    uint16_t* w16;                 // [RC_NPARAM] bf16 in fragment order
+    uint16_t* wT16;                // the transposed matrices in fragment order, for backward
     float* w32;                    // master copy
     float* wGrad;
     float* wM;
@@ -54,7 +76,7 @@ struct DNrcNet {
 // Per-batch activation buffers of training, `tiles` = samples / 16. The *T
 // buffers are tile-transposed bf16: [tile][feature][16 samples].
 struct DNrcActs {
-    uint16_t* x0;                  // [samples][48] bf16, sample-major
+    uint32_t* x0;                  // [RC_LEVELS][samples] a level's two bf16 features
     uint16_t* x0T;                 // [tile][48][16]
     uint16_t* hT[3];               // [tile][64][16]
     uint16_t* dzT[3];              // [tile][64][16]
@@ -68,10 +90,8 @@ struct DNrcAdam {
     float emaScale;                // 1 / (1 - d^t): debiasing of E (which starts at 0)
 };
 
-int dn_rc_encode(const DNrcNet& net, const float* samples, uint32_t n, uint16_t* x0, hipStream_t stream);
-// pred: float4 per row (3 outputs, the row's valid flag; 1 without samples).
-int dn_rc_forward(const DNrcNet& net, const uint16_t* x0, const float* samples, uint32_t n, float* pred,
-                  hipStream_t stream);
+// pred: float4 per row (3 outputs plus the row's exact term, the row's valid flag).
+int dn_rc_predict(const DNrcNet& net, const float* samples, uint32_t n, float* pred, hipStream_t stream);
 // A second stream for training: the weight gradients run on it beside the
 // table gradients (`fork` and `join` order it after the MLP and before Adam).
 struct DNrcSide {
@@ -81,13 +101,6 @@ struct DNrcSide {
 // side: null runs every kernel on `stream`.
 int dn_rc_train(const DNrcNet& net, const float* samples, uint32_t n, const DNrcActs& a, hipStream_t stream,
                 const DNrcSide* side = nullptr);
-// Allocation-free prediction: dn_rc_encode + dn_rc_forward with the encoded rows
-// in the fixed per-device scratch array of rcache.hip (at most
-// DNX_RC_NOALLOC_MAX_SAMPLES rows) on device `device`. dn_noalloc_init (called
-// by DN_init) looks up every device's address of that array first.
-bool dn_noalloc_init();
-int dn_rc_predict_noalloc(const DNrcNet& net, int device, const float* samples, uint32_t n, float* pred,
-                          hipStream_t stream);
 int dn_rc_adam(const DNrcNet& net, const DNrcAdam& opt, hipStream_t stream);
 // `batches` batches of n training samples, batch k drawn with seed + k * seedStride
 int dn_rc_samples(const DNlightParams& p, uint32_t maxRequests, uint32_t n, uint32_t batches, uint32_t seed,

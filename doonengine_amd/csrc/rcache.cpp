@@ -14,7 +14,6 @@ void dn_msg(DNmessageType type, DNmessageSeverity sev, const char* fmt, ...);
 struct DNXradianceCache {
     DNvolume* vol = nullptr;
     hipStream_t stream = nullptr;
-    int device = 0;               // the device its buffers live on (current at creation)
     DNXrcConfig cfg;
     DNrcNet net;
     DNrcActs acts;
@@ -24,7 +23,6 @@ struct DNXradianceCache {
     const float* lastSamplesPtr = nullptr;   // the last step's rows in dSamples
     uint32_t lastSamples = 0;
     float* dQuery = nullptr;      // query rows for predictions
-    uint16_t* dQueryX0 = nullptr;
     size_t queryCap = 0;
     uint32_t adamStep = 0;
     double emaKeep = 1.0;         // product of the average's decays so far (its debiasing)
@@ -82,8 +80,12 @@ bool upload_params(DNXradianceCache* rc, const float* w, const float* tab)
 {
     const size_t tf = table_floats(rc);
     std::vector<uint16_t> w16(RC_NPARAM), wT16(RC_NPARAM);
-    for(int i = 0; i < RC_NPARAM; i++) w16[i] = host_bf16(w[i]);
-    for(uint32_t i = 0; i < RC_NPARAM; i++) wT16[rc_transposed_index(i)] = w16[i];
+    for(uint32_t i = 0; i < RC_NPARAM; i++)
+    {
+        uint32_t f, t;
+        rc_fragment_positions(i, f, t);
+        w16[f] = wT16[t] = host_bf16(w[i]);
+    }
     std::vector<uint32_t> t16(tf / 2);
     for(size_t i = 0; i < tf / 2; i++) t16[i] = host_bf16(tab[2 * i]) | ((uint32_t)host_bf16(tab[2 * i + 1]) << 16);
     DNrcNet& n = rc->net;
@@ -111,7 +113,7 @@ bool ensure_train(DNXradianceCache* rc, uint32_t n)
     hipStreamSynchronize(rc->stream);
     dfree(a.x0); dfree(a.x0T); dfree(a.dyT); dfree(a.denc);
     for(int i = 0; i < 3; i++) { dfree(a.hT[i]); dfree(a.dzT[i]); }
-    bool g = dev(&a.x0, (size_t)n * RC_IN, "activations") && dev(&a.x0T, (size_t)n * RC_IN, "activations") &&
+    bool g = dev(&a.x0, (size_t)n * RC_LEVELS, "activations") && dev(&a.x0T, (size_t)n * RC_IN, "activations") &&
              dev(&a.dyT, (size_t)n * RC_OUT, "activations") && dev(&a.denc, (size_t)n * RC_ENC, "activations");
     for(int i = 0; g && i < 3; i++)
         g = dev(&a.hT[i], (size_t)n * RC_W, "activations") && dev(&a.dzT[i], (size_t)n * RC_W, "activations");
@@ -136,8 +138,7 @@ bool ensure_query(DNXradianceCache* rc, size_t n)
     if(n <= rc->queryCap) return true;
     hipStreamSynchronize(rc->stream);
     dfree(rc->dQuery);
-    dfree(rc->dQueryX0);
-    bool g = dev(&rc->dQuery, n * RC_SAMPLE, "queries") && dev(&rc->dQueryX0, n * RC_IN, "queries");
+    const bool g = dev(&rc->dQuery, n * RC_SAMPLE, "queries");
     rc->queryCap = g ? n : 0;
     return g;
 }
@@ -215,7 +216,6 @@ extern "C" void DNX_rc_destroy(DNXradianceCache* rc)
     dfree(rc->dSamples); dfree(a.x0); dfree(a.x0T); dfree(a.dyT); dfree(a.denc);
     for(int i = 0; i < 3; i++) { dfree(a.hT[i]); dfree(a.dzT[i]); }
     dfree(rc->dQuery);
-    dfree(rc->dQueryX0);
     delete rc;
 }
 
@@ -249,7 +249,6 @@ extern "C" DNXradianceCache* DNX_rc_create(DNvolume* vol, const DNXrcConfig* con
         if(rc->side.join) hipEventDestroy(rc->side.join);
         rc->side = DNrcSide{nullptr, nullptr, nullptr};
     }
-    if(hipGetDevice(&rc->device) != hipSuccess) rc->device = 0;
     if(c.extent <= 0.0f)
     {
         uint32_t m = vol->mapSize.x > vol->mapSize.y ? vol->mapSize.x : vol->mapSize.y;
@@ -334,10 +333,7 @@ extern "C" bool DNX_rc_train_samples(DNXradianceCache* rc, const float* samples,
 extern "C" bool DNX_rc_predict_samples(DNXradianceCache* rc, const float* samples, uint32_t n, float* out)
 {
     if(!rc || !samples || !out || n == 0 || (n & 15u)) return false;
-    if(!ensure_query(rc, n)) return false;
-    const DNrcNet inf = infer_net(rc);
-    return dn_rc_encode(inf, samples, n, rc->dQueryX0, rc->stream) == 0 &&
-           dn_rc_forward(inf, rc->dQueryX0, samples, n, out, rc->stream) == 0;
+    return dn_rc_predict(infer_net(rc), samples, n, out, rc->stream) == 0;
 }
 
 extern "C" bool DNX_rc_predict_samples_noalloc(DNXradianceCache* rc, const float* samples, uint32_t n, float* out)
@@ -350,12 +346,14 @@ extern "C" bool DNX_rc_predict_samples_noalloc(DNXradianceCache* rc, const float
                DNX_RC_NOALLOC_MAX_SAMPLES);
         return false;
     }
-    const int e = dn_rc_predict_noalloc(infer_net(rc), rc->device, samples, n, out, rc->stream);
-    if(e == (int)hipErrorNotInitialized)
+    if(!dn_initialised())
+    {
         dn_msg(DN_MESSAGE_GPU_MEMORY, DN_MESSAGE_ERROR,
-               "radiance cache: no scratch array on device %d (DN_init was not called)", rc->device);
-    else if(e)
-        dn_msg(DN_MESSAGE_SHADER, DN_MESSAGE_ERROR, "radiance cache: allocation-free prediction failed (%d)", e);
+               "radiance cache: DN_init was not called before the allocation-free prediction");
+        return false;
+    }
+    const int e = dn_rc_predict(infer_net(rc), samples, n, out, rc->stream);
+    if(e) dn_msg(DN_MESSAGE_SHADER, DN_MESSAGE_ERROR, "radiance cache: allocation-free prediction failed (%d)", e);
     return e == 0;
 }
 
@@ -406,10 +404,8 @@ extern "C" bool DNX_rc_predict_requests(DNXradianceCache* rc, float* out, size_t
     size_t slots = (size_t)requestCapacity * 32u;
     if(slots == 0) return true;
     if(slots > 0xFFFFFFF0u || !ensure_query(rc, slots)) return false;
-    const DNrcNet inf = infer_net(rc);
     return dn_rc_gather(p, (uint32_t)slots, rc->dQuery, rc->stream) == 0 &&
-           dn_rc_encode(inf, rc->dQuery, (uint32_t)slots, rc->dQueryX0, rc->stream) == 0 &&
-           dn_rc_forward(inf, rc->dQueryX0, rc->dQuery, (uint32_t)slots, out, rc->stream) == 0;
+           dn_rc_predict(infer_net(rc), rc->dQuery, (uint32_t)slots, out, rc->stream) == 0;
 }
 
 extern "C" bool DNX_rc_reference(DNXradianceCache* rc, double* acc, size_t requestCapacity, uint32_t samplesPerVoxel,

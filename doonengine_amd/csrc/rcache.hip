@@ -19,25 +19,24 @@
 #include "rc_internal.h"
 #include "doon/doon.h"
 
-#include <mutex>
-#include <vector>
-
 namespace {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint16_t f2bf(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    if((u & 0x7F800000u) == 0x7F800000u) return (uint16_t)((u >> 16) | ((u & 0xFFFFu) ? 0x40u : 0u));
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-__device__ __forceinline__ float bf2f(uint32_t h) { return __uint_as_float(h << 16); }
-
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 hwbf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
+
+// Nearest-even bfloat16: v_cvt_pk_bf16_f32, which agrees with rounding the bits
+// in integer arithmetic on every float that is not a NaN (NaNs stay NaNs).
+__device__ __forceinline__ uint32_t f2bf2(float lo, float hi)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, hwbf16x2));
+}
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+__device__ __forceinline__ float bf2f(uint32_t h) { return __uint_as_float(h << 16); }
 
 __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c)
 {
@@ -49,47 +48,44 @@ __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c)
 // 4 of A1, and likewise for B, so A and B pair the same 32 k-values (a
 // permutation of the K = 32 block, which leaves the dot product a sum over
 // the same terms) and two C-layout tiles feed B without any shuffle.
-__device__ __forceinline__ f32x4 mfma32(bf16x4 a0, bf16x4 a1, bf16x4 b0, bf16x4 b1, f32x4 c)
+__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x4 b0, bf16x4 b1, f32x4 c)
 {
-    const s16x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
     const s16x8 b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                   0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 __device__ __forceinline__ bf16x4 ld_bf16x4(const uint16_t* p)
 {
-    uint2 v = *reinterpret_cast<const uint2*>(p);
-    bf16x4 r;
-    r[0] = (short)(v.x & 0xFFFFu); r[1] = (short)(v.x >> 16);
-    r[2] = (short)(v.y & 0xFFFFu); r[3] = (short)(v.y >> 16);
-    return r;
+    return __builtin_bit_cast(bf16x4, *reinterpret_cast<const uint2*>(p));
 }
 
-// A operand of a 16x16 block of a row-major bf16 matrix M (leading dimension
-// ld) at (row0, k0): lane holds M[row0 + (lane & 15)][k0 + 4 * (lane >> 4) + j].
-__device__ __forceinline__ bf16x4 a_rows(const uint16_t* M, uint32_t ld, uint32_t row0, uint32_t k0, uint32_t lane)
+// A operands of a matrix in fragment order (rc_fragment_index): `block` is the
+// element offset of a 16x32 or 16x16 block.
+__device__ __forceinline__ bf16x8 a_frag32(const uint16_t* block, uint32_t lane)
 {
-    return ld_bf16x4(M + (row0 + (lane & 15u)) * ld + k0 + 4u * (lane >> 4));
+    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(block + lane * 8u));
+}
+__device__ __forceinline__ bf16x4 a_frag16(const uint16_t* block, uint32_t lane)
+{
+    return ld_bf16x4(block + lane * 4u);
+}
+
+__device__ __forceinline__ bf16x4 to_bf16(f32x4 c)
+{
+    return __builtin_bit_cast(bf16x4, make_uint2(f2bf2(c[0], c[1]), f2bf2(c[2], c[3])));
 }
 
 __device__ __forceinline__ bf16x4 relu_bf16(f32x4 c)
 {
-    bf16x4 r;
-    for(int i = 0; i < 4; i++) r[i] = (short)f2bf(c[i] > 0.0f ? c[i] : 0.0f);
-    return r;
+    for(int i = 0; i < 4; i++) c[i] = c[i] > 0.0f ? c[i] : 0.0f;
+    return to_bf16(c);
 }
 
 // Gradient through ReLU: keep d where the layer output h (bf16) is positive.
 __device__ __forceinline__ bf16x4 relu_grad(f32x4 d, bf16x4 h)
 {
-    bf16x4 r;
-    for(int i = 0; i < 4; i++)
-    {
-        uint16_t hb = (uint16_t)h[i];
-        r[i] = (short)((hb != 0u && !(hb & 0x8000u)) ? f2bf(d[i]) : 0u);
-    }
-    return r;
+    for(int i = 0; i < 4; i++) d[i] = h[i] > 0 ? d[i] : 0.0f;     // bits of h: not -0, +0 or negative
+    return to_bf16(d);
 }
 
 // Stores a C-layout bf16 tile of feature block fb into a tile-transposed
@@ -106,22 +102,29 @@ __device__ __forceinline__ void store_T(uint16_t* T, uint32_t F, uint32_t tile, 
 // ---------------------------------------------------------------------------
 // encoding
 
-// The cell of a level that holds a position: its lower corner g and the
-// position's fractions f inside it.
+// A position over the extent, clamped to the unit cube.
+struct UnitPos { float v[3]; };
+
+__device__ __forceinline__ UnitPos unit_pos(const DNrcNet& net, const float* pos)
+{
+    UnitPos u;
+    for(int a = 0; a < 3; a++) u.v[a] = fminf(fmaxf(pos[a] / net.extent, 0.0f), 1.0f);
+    return u;
+}
+
+// The cell of a level of resolution N that holds a position: its lower corner
+// g and the position's fractions f inside it.
 struct LevelCell {
     uint32_t g[3];
     float f[3];
 };
 
-__device__ __forceinline__ LevelCell level_cell(const DNrcNet& net, uint32_t l, const float* pos)
+__device__ __forceinline__ LevelCell level_cell(uint32_t N, const UnitPos& u)
 {
     LevelCell c;
-    const uint32_t N = net.res[l];
     for(int a = 0; a < 3; a++)
     {
-        float x = pos[a] / net.extent;
-        x = fminf(fmaxf(x, 0.0f), 1.0f);
-        float s = x * (float)N + 0.5f;
+        float s = u.v[a] * (float)N + 0.5f;
         float fl = floorf(s);
         c.g[a] = (uint32_t)fl;
         c.f[a] = s - fl;
@@ -131,51 +134,71 @@ __device__ __forceinline__ LevelCell level_cell(const DNrcNet& net, uint32_t l, 
 
 // Corner k (bit 0: x + 1, bit 1: y + 1, bit 2: z + 1) of a cell: its table
 // entry (dense index, or the spatial hash) and its trilinear weight.
-__device__ __forceinline__ void cell_corner(const DNrcNet& net, uint32_t l, const LevelCell& c, uint32_t k,
-                                            uint32_t& idx, float& w)
+__device__ __forceinline__ uint32_t corner_index(uint32_t N, bool dense, uint32_t mask, const LevelCell& c, uint32_t k)
 {
-    const uint32_t T = 1u << net.log2T;
-    const bool dense = (net.denseMask >> l) & 1u;
-    const uint32_t S = net.res[l] + 2u;
+    const uint32_t S = N + 2u;
     const uint32_t cx = c.g[0] + (k & 1u), cy = c.g[1] + ((k >> 1) & 1u), cz = c.g[2] + ((k >> 2) & 1u);
     const uint32_t i = dense ? cx + cy * S + cz * S * S : (cx * 1u) ^ (cy * 2654435761u) ^ (cz * 805459861u);
-    idx = i & (T - 1u);
-    w = ((k & 1u) ? c.f[0] : 1.0f - c.f[0]) * ((k & 2u) ? c.f[1] : 1.0f - c.f[1]) *
-        ((k & 4u) ? c.f[2] : 1.0f - c.f[2]);
+    return i & mask;
 }
 
-// One thread per (sample, level): the level's two features into x0, level 0
-// also the normal, albedo and zero padding. (Two lanes per pair, each
-// gathering the corners of one x offset so that a load instruction takes a
-// sample's two x-neighbour entries at once, measured 52.7 against 46.9 us per
-// 2^17 samples: unlike the atomics, these gathers are not bound by the cache
-// lines an instruction touches.)
-__global__ __launch_bounds__(256) void k_rc_encode(DNrcNet net, const float* samples, uint32_t n, uint16_t* x0)
+__device__ __forceinline__ float corner_weight(const LevelCell& c, uint32_t k)
 {
-    const uint32_t g = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t s = g >> 4, l = g & 15u;
-    if(s >= n) return;
-    const float* sp = samples + (size_t)s * RC_SAMPLE;
-    const LevelCell cell = level_cell(net, l, sp);
-    const uint32_t* tab = net.tab16 + ((size_t)l << net.log2T);
-    uint32_t idx[8];
-    float w[8];
-    for(uint32_t k = 0; k < 8u; k++) cell_corner(net, l, cell, k, idx[k], w[k]);
+    return ((k & 1u) ? c.f[0] : 1.0f - c.f[0]) * ((k & 2u) ? c.f[1] : 1.0f - c.f[1]) *
+           ((k & 4u) ? c.f[2] : 1.0f - c.f[2]);
+}
+
+// A level's two features of a position, as bf16 (first feature in the low half).
+// `level` is the entry index at which the level's table starts. KIND: every lane
+// of the wave is at a dense level (1), at a hashed one (2), or either (0).
+template <int KIND>
+__device__ __forceinline__ uint32_t encode_level(const uint32_t* tab, uint32_t level, uint32_t N, bool dense,
+                                                 uint32_t mask, const UnitPos& u)
+{
+    const LevelCell c = level_cell(N, u);
+    if(KIND) dense = KIND == 1;
+    // corner (x, y, z): x + y S + z S^2, or x ^ y P ^ z P' mod T
+    const uint32_t S = N + 2u;
+    const uint32_t my = dense ? S : 2654435761u, mz = dense ? S * S : 805459861u;
+    const uint32_t y0 = c.g[1] * my, z0 = c.g[2] * mz;
     uint32_t e[8];
-    for(uint32_t k = 0; k < 8u; k++) e[k] = tab[idx[k]];        // all eight gathers in flight at once
-    float a0 = 0.0f, a1 = 0.0f;
+    #pragma unroll
     for(uint32_t k = 0; k < 8u; k++)
     {
-        a0 += w[k] * bf2f(e[k] & 0xFFFFu);
-        a1 += w[k] * bf2f(e[k] >> 16);
+        const uint32_t x = c.g[0] + (k & 1u), y = (k & 2u) ? y0 + my : y0, z = (k & 4u) ? z0 + mz : z0;
+        const uint32_t i = (dense ? x + (y + z) : x ^ (y ^ z)) & mask;
+        // a 32-bit byte offset (the tables hold at most 2^28 entries)
+        e[k] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(tab) + ((level + i) << 2));
     }
-    uint16_t* row = x0 + (size_t)s * RC_IN;
-    row[2 * l] = f2bf(a0);
-    row[2 * l + 1] = f2bf(a1);
-    if(l == 0)
+    float a0 = 0.0f, a1 = 0.0f;
+    #pragma unroll
+    for(uint32_t k = 0; k < 8u; k++)
     {
-        for(int i = 0; i < 6; i++) row[RC_ENC + i] = f2bf(sp[3 + i]);
-        for(int i = RC_ENC + 6; i < RC_IN; i++) row[i] = 0;
+        const float w = corner_weight(c, k);
+        a0 += w * bf2f(e[k] & 0xFFFFu);
+        a1 += w * bf2f(e[k] >> 16);
+    }
+    return f2bf2(a0, a1);
+}
+
+// Encoding of many rows, one level per wave: a lane takes one sample at levels
+// 15 - b and b, b = blockIdx mod 8. Workgroups go to the 8 XCDs in turn, so each
+// XCD's 4 MiB L2 serves one fine and one coarse level (2 MiB each at 2^19
+// entries) instead of all sixteen, and on the coarse levels neighbouring rows
+// of a wave share their entries' lines. Level-major output: 256-byte stores.
+__global__ __launch_bounds__(256) void k_rc_encode(DNrcNet net, const float* samples, uint32_t n, uint32_t* x0)
+{
+    const uint32_t b = blockIdx.x & 7u;
+    const uint32_t s = (blockIdx.x >> 3) * 256u + threadIdx.x;
+    if(s >= n) return;
+    const UnitPos u = unit_pos(net, samples + (size_t)s * RC_SAMPLE);
+    const uint32_t mask = (1u << net.log2T) - 1u;
+    for(uint32_t i = 0; i < 2u; i++)
+    {
+        const uint32_t l = i ? b : RC_LEVELS - 1u - b;
+        const bool dense = (net.denseMask >> l) & 1u;            // the same for the whole wave
+        x0[(size_t)l * n + s] = dense ? encode_level<1>(net.tab16, l << net.log2T, net.res[l], true, mask, u)
+                                      : encode_level<2>(net.tab16, l << net.log2T, net.res[l], false, mask, u);
     }
 }
 
@@ -207,101 +230,172 @@ __global__ __launch_bounds__(256) void k_rc_table_grad(DNrcNet net, const float*
     const float d = denc[(size_t)s * RC_ENC + 2u * l + f];
     if(d == 0.0f) return;                                       // adding +-0 changes no sum
     float* gt = net.tabGrad + ((size_t)l << net.log2T) * 2u;
-    const LevelCell cell = level_cell(net, l, samples + (size_t)s * RC_SAMPLE);
+    const uint32_t N = net.res[l], mask = (1u << net.log2T) - 1u;
+    const bool dense = (net.denseMask >> l) & 1u;
+    const LevelCell cell = level_cell(N, unit_pos(net, samples + (size_t)s * RC_SAMPLE));
     for(uint32_t j = 0; j < 4u; j++)
     {
-        uint32_t idx;
-        float wt;
-        cell_corner(net, l, cell, (j << 1) | xb, idx, wt);
-        atomicAdd(gt + 2u * idx + f, wt * d);
+        const uint32_t k = (j << 1) | xb;
+        atomicAdd(gt + 2u * corner_index(N, dense, mask, cell, k) + f, corner_weight(cell, k) * d);
     }
 }
 
 // ---------------------------------------------------------------------------
-// MLP: forward (and, with TRAIN, backward) over 16-sample tiles, one tile per
-// wave at a time. Weights (and with TRAIN their transposes) staged in LDS.
+// MLP over 16-sample tiles. Weights in fragment order, staged in LDS by 16-byte
+// pieces.
 
-template <bool TRAIN>
-__global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const uint16_t* x0, const float* samples, uint32_t n,
-                                                float invB, float* pred, DNrcActs acts)
+__device__ __forceinline__ void stage_weights(uint16_t* lds, const uint16_t* w, uint32_t threads)
 {
-    __shared__ __align__(16) uint16_t W[RC_NPARAM];
-    __shared__ __align__(16) uint16_t WT[TRAIN ? RC_NPARAM : 8];
-    // the weights, and for the backward pass their transposes (W0^T 48x64,
-    // W1^T, W2^T 64x64, W3^T 64x16, same offsets; written by the Adam step),
-    // staged in 16-byte pieces
-    for(uint32_t i = threadIdx.x; i < RC_NPARAM / 8u; i += 256u)
+    for(uint32_t i = threadIdx.x; i < RC_NPARAM / 8u; i += threads)
+        reinterpret_cast<uint4*>(lds)[i] = reinterpret_cast<const uint4*>(w)[i];
+}
+
+// A row's third 16-feature input block: normal, albedo, zeros.
+__device__ __forceinline__ bf16x4 surface_input(const float* row, uint32_t q)
+{
+    f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+    if(q == 0u) x = f32x4{row[3], row[4], row[5], row[6]};
+    else if(q == 1u) x = f32x4{row[7], row[8], 0.0f, 0.0f};
+    return to_bf16(x);
+}
+
+// A lane's features 4 q + 0..3 of a 16-feature block: two levels' words.
+__device__ __forceinline__ bf16x4 level_input(uint32_t even, uint32_t odd)
+{
+    return __builtin_bit_cast(bf16x4, make_uint2(even, odd));
+}
+
+__device__ __forceinline__ void load_input(const uint32_t* x0, uint32_t n, uint32_t sm, const float* row, uint32_t q,
+                                           bf16x4 xin[3])
+{
+    for(uint32_t b = 0; b < 2u; b++)
     {
-        reinterpret_cast<uint4*>(W)[i] = reinterpret_cast<const uint4*>(net.w16)[i];
-        if(TRAIN) reinterpret_cast<uint4*>(WT)[i] = reinterpret_cast<const uint4*>(net.wT16)[i];
+        const uint32_t* p = x0 + (size_t)(8u * b + 2u * q) * n + sm;
+        xin[b] = level_input(p[0], p[n]);
     }
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t tiles = n / 16u;
-    for(uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6); tile < tiles; tile += gridDim.x * 4u)
-    {
-        const uint32_t s0 = tile * 16u;
-        const uint32_t sm = s0 + (lane & 15u);
-        bf16x4 xin[3];
-        for(uint32_t ks = 0; ks < 3; ks++) xin[ks] = ld_bf16x4(x0 + (size_t)sm * RC_IN + ks * 16u + 4u * (lane >> 4));
-        bf16x4 h[3][4];
-        f32x4 acc[4];
+    xin[2] = surface_input(row, q);
+}
+
+// One tile. The first layer's third input block is a 16x16x16 product on top of
+// the 16x16x32 one. Right behind it, that product has added to an unfinished
+// accumulator (wrong elements 0 and 1 of the four: the two instructions take
+// different numbers of passes, and the compiler puts no wait between them), so
+// all four row blocks go through the K = 32 instruction first: three of them lie
+// between a block's two products.
+__device__ __forceinline__ void mlp_forward(const uint16_t* W, uint32_t lane, const bf16x4 xin[3], bf16x4 h[3][4],
+                                            f32x4& y)
+{
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x4 c[4];
+    f32x4 acc[4];
+    #pragma unroll
+    for(uint32_t mb = 0; mb < 4; mb++) c[mb] = a_frag16(W + RC_OFF_W0 + mb * 768u + 512u, lane);
+    #pragma unroll
+    for(uint32_t mb = 0; mb < 4; mb++)
+        acc[mb] = mfma32(a_frag32(W + RC_OFF_W0 + mb * 768u, lane), xin[0], xin[1], zero);
+    __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+    for(uint32_t mb = 0; mb < 4; mb++) acc[mb] = mfma16(c[mb], xin[2], acc[mb]);
+    __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+    for(uint32_t mb = 0; mb < 4; mb++) h[0][mb] = relu_bf16(acc[mb]);
+    #pragma unroll
+    for(uint32_t layer = 1; layer < 3; layer++)
+        #pragma unroll
         for(uint32_t mb = 0; mb < 4; mb++)
         {
-            acc[mb] = mfma32(a_rows(W + RC_OFF_W0, 48, mb * 16u, 0u, lane), a_rows(W + RC_OFF_W0, 48, mb * 16u, 16u, lane),
-                             xin[0], xin[1], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-            acc[mb] = mfma16(a_rows(W + RC_OFF_W0, 48, mb * 16u, 32u, lane), xin[2], acc[mb]);
+            const uint16_t* w = W + (layer == 1 ? RC_OFF_W1 : RC_OFF_W2) + mb * 1024u;
+            const f32x4 d = mfma32(a_frag32(w, lane), h[layer - 1][0], h[layer - 1][1], zero);
+            h[layer][mb] = relu_bf16(mfma32(a_frag32(w + 512, lane), h[layer - 1][2], h[layer - 1][3], d));
         }
-        for(uint32_t mb = 0; mb < 4; mb++) h[0][mb] = relu_bf16(acc[mb]);
-        for(uint32_t layer = 1; layer < 3; layer++)
+    y = mfma32(a_frag32(W + RC_OFF_W3, lane), h[2][0], h[2][1], zero);
+    y = mfma32(a_frag32(W + RC_OFF_W3 + 512, lane), h[2][2], h[2][3], y);
+}
+
+// Predictions: each lane encodes the four levels whose features it feeds to the
+// first layer, so there is one launch and no pass over encoded rows, and no
+// scratch memory that calls would share. Bound by the 128 table gathers a row
+// needs (2^20 rows: 0.73 T gathers/s where the tables exceed the L2s, 1.05 T/s
+// where they fit). Against encoding all rows in a launch of their own (a level
+// per wave, each XCD two levels) 5.7 against 7.5 us at 1008 rows, 17.6 against
+// 22.6 at 65 536 and 181 against 202 at 10^6 (2^19 entries); one row per
+// 16 lanes with the weights' LDS reads in bank conflict took 13.1, 44.9 and 360.
+__global__ __launch_bounds__(256) void k_rc_predict(DNrcNet net, const float* samples, uint32_t n, float* pred)
+{
+    __shared__ __align__(16) uint16_t W[RC_NPARAM];
+    __shared__ uint32_t res[RC_LEVELS];
+    stage_weights(W, net.w16, 256u);
+    if(threadIdx.x < RC_LEVELS) res[threadIdx.x] = net.res[threadIdx.x];
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u, q = lane >> 4;
+    const uint32_t tiles = n / 16u, mask = (1u << net.log2T) - 1u;
+    for(uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6); tile < tiles; tile += gridDim.x * 4u)
+    {
+        const uint32_t sm = tile * 16u + (lane & 15u);
+        const float* row = samples + (size_t)sm * RC_SAMPLE;
+        bf16x4 xin[3], h[3][4];
+        f32x4 y;
+        const UnitPos u = unit_pos(net, row);
+        uint32_t e[4];
+        #pragma unroll
+        for(uint32_t i = 0; i < 4u; i++)
         {
-            const uint16_t* Wl = W + (layer == 1 ? RC_OFF_W1 : RC_OFF_W2);
-            for(uint32_t mb = 0; mb < 4; mb++)
-            {
-                acc[mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                for(uint32_t ks = 0; ks < 4; ks += 2)
-                    acc[mb] = mfma32(a_rows(Wl, 64, mb * 16u, ks * 16u, lane), a_rows(Wl, 64, mb * 16u, ks * 16u + 16u, lane),
-                                     h[layer - 1][ks], h[layer - 1][ks + 1], acc[mb]);
-            }
-            for(uint32_t mb = 0; mb < 4; mb++) h[layer][mb] = relu_bf16(acc[mb]);
+            // the wave's levels at this step: 8 (i / 2) + 2 q + i mod 2, q = 0..3
+            const uint32_t l = 8u * (i >> 1) + 2u * q + (i & 1u);
+            const uint32_t kinds = (net.denseMask >> (8u * (i >> 1) + (i & 1u))) & 0x55u;
+            if(kinds == 0x55u) e[i] = encode_level<1>(net.tab16, l << net.log2T, res[l], true, mask, u);
+            else if(kinds == 0u) e[i] = encode_level<2>(net.tab16, l << net.log2T, res[l], false, mask, u);
+            else e[i] = encode_level<0>(net.tab16, l << net.log2T, res[l], (net.denseMask >> l) & 1u, mask, u);
         }
-        f32x4 y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        for(uint32_t ks = 0; ks < 4; ks += 2)
-            y = mfma32(a_rows(W + RC_OFF_W3, 64, 0, ks * 16u, lane), a_rows(W + RC_OFF_W3, 64, 0, ks * 16u + 16u, lane),
-                       h[2][ks], h[2][ks + 1], y);
-        // y: lane < 16 holds outputs 0..3 of sample s0 + lane (3 used)
-        if(!TRAIN)
-        {
-            if(lane < 16u && sm < n)
-            {
-                // a row may carry an exactly computed term (direct light) in 13..15
-                const float* sp = samples ? samples + (size_t)sm * RC_SAMPLE : nullptr;
-                const float valid = sp ? sp[12] : 1.0f;
-                const float b0 = sp ? sp[13] : 0.0f, b1 = sp ? sp[14] : 0.0f, b2 = sp ? sp[15] : 0.0f;
-                reinterpret_cast<float4*>(pred)[sm] = make_float4(y[0] + b0, y[1] + b1, y[2] + b2, valid);
-            }
-            continue;
-        }
+        xin[0] = level_input(e[0], e[1]);
+        xin[1] = level_input(e[2], e[3]);
+        xin[2] = surface_input(row, q);
+        // the weights stay in LDS: held in registers over the tiles (96 of them)
+        // they would halve the waves that hide the gathers
+        asm volatile("" ::: "memory");
+        mlp_forward(W, lane, xin, h, y);
+        // y: lane < 16 holds outputs 0..3 of the tile's sample `lane` (3 used);
+        // a row may carry an exactly computed term (direct light) in 13..15
+        if(lane < 16u)
+            reinterpret_cast<float4*>(pred)[sm] =
+                make_float4(y[0] + row[13], y[1] + row[14], y[2] + row[15], row[12]);
+    }
+}
+
+// Forward and backward of training, one tile per wave at a time.
+__global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const float* samples, uint32_t n, float invB,
+                                                DNrcActs acts)
+{
+    __shared__ __align__(16) uint16_t W[RC_NPARAM];
+    __shared__ __align__(16) uint16_t WT[RC_NPARAM];
+    stage_weights(W, net.w16, 256u);
+    stage_weights(WT, net.wT16, 256u);
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u, q = lane >> 4;
+    const uint32_t tiles = n / 16u;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    for(uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6); tile < tiles; tile += gridDim.x * 4u)
+    {
+        const uint32_t sm = tile * 16u + (lane & 15u);
+        const float* row = samples + (size_t)sm * RC_SAMPLE;
+        bf16x4 xin[3], h[3][4];
+        f32x4 y;
+        load_input(acts.x0, n, sm, row, q, xin);
+        mlp_forward(W, lane, xin, h, y);
         for(uint32_t ks = 0; ks < 3; ks++) store_T(acts.x0T, RC_IN, tile, ks, xin[ks], lane);
         for(uint32_t layer = 0; layer < 3; layer++)
             for(uint32_t mb = 0; mb < 4; mb++) store_T(acts.hT[layer], RC_W, tile, mb, h[layer][mb], lane);
         // dL/dy = (y - t) / B for valid samples
-        f32x4 dy = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if(lane < 16u)
-        {
-            const float* sp = samples + (size_t)sm * RC_SAMPLE;
-            if(sp[12] != 0.0f)
-                for(int i = 0; i < 3; i++) dy[i] = (y[i] - sp[9 + i]) * invB;
-        }
-        bf16x4 dyb;
-        for(int i = 0; i < 4; i++) dyb[i] = (short)f2bf(dy[i]);
+        f32x4 dy = zero;
+        if(lane < 16u && row[12] != 0.0f)
+            for(int i = 0; i < 3; i++) dy[i] = (y[i] - row[9 + i]) * invB;
+        const bf16x4 dyb = to_bf16(dy);
         store_T(acts.dyT, RC_OUT, tile, 0, dyb, lane);
         // dH3^T = W3^T dY^T (K = 16 outputs), then through the ReLUs
         bf16x4 dz[4];
         for(uint32_t mb = 0; mb < 4; mb++)
         {
-            f32x4 d = mfma16(a_rows(WT + RC_OFF_W3, 16, mb * 16u, 0, lane), dyb, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-            dz[mb] = relu_grad(d, h[2][mb]);
+            dz[mb] = relu_grad(mfma16(a_frag16(WT + RC_OFF_W3 + mb * 256u, lane), dyb, zero), h[2][mb]);
             store_T(acts.dzT[2], RC_W, tile, mb, dz[mb], lane);
         }
         for(int layer = 1; layer >= 0; layer--)
@@ -311,10 +405,8 @@ __global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const uint16_t* x0,
             bf16x4 nz[4];
             for(uint32_t mb = 0; mb < 4; mb++)
             {
-                f32x4 d = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                for(uint32_t ks = 0; ks < 4; ks += 2)
-                    d = mfma32(a_rows(WTl, 64, mb * 16u, ks * 16u, lane), a_rows(WTl, 64, mb * 16u, ks * 16u + 16u, lane),
-                               dz[ks], dz[ks + 1], d);
+                f32x4 d = mfma32(a_frag32(WTl + mb * 1024u, lane), dz[0], dz[1], zero);
+                d = mfma32(a_frag32(WTl + mb * 1024u + 512u, lane), dz[2], dz[3], d);
                 nz[mb] = relu_grad(d, h[layer][mb]);
                 store_T(acts.dzT[layer], RC_W, tile, mb, nz[mb], lane);
             }
@@ -323,11 +415,9 @@ __global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const uint16_t* x0,
         // dX0^T = W0^T dZ1^T, encoded features only (rows 0..31)
         for(uint32_t mb = 0; mb < 2; mb++)
         {
-            f32x4 d = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            for(uint32_t ks = 0; ks < 4; ks += 2)
-                d = mfma32(a_rows(WT + RC_OFF_W0, 64, mb * 16u, ks * 16u, lane),
-                           a_rows(WT + RC_OFF_W0, 64, mb * 16u, ks * 16u + 16u, lane), dz[ks], dz[ks + 1], d);
-            reinterpret_cast<float4*>(acts.denc + (size_t)sm * RC_ENC + mb * 16u + 4u * (lane >> 4))[0] =
+            f32x4 d = mfma32(a_frag32(WT + RC_OFF_W0 + mb * 1024u, lane), dz[0], dz[1], zero);
+            d = mfma32(a_frag32(WT + RC_OFF_W0 + mb * 1024u + 512u, lane), dz[2], dz[3], d);
+            reinterpret_cast<float4*>(acts.denc + (size_t)sm * RC_ENC + mb * 16u + 4u * q)[0] =
                 make_float4(d[0], d[1], d[2], d[3]);
         }
     }
@@ -408,9 +498,10 @@ __global__ __launch_bounds__(256) void k_rc_adam(DNrcNet net, DNrcAdam o, size_t
         adam_one(w, net.wGrad[i], m, v, o);
         net.w32[i] = w; net.wM[i] = m; net.wV[i] = v;
         net.wGrad[i] = 0.0f;
-        net.w16[i] = f2bf(w);
-        net.wT16[rc_transposed_index((uint32_t)i)] = f2bf(w);
-        net.wE16[i] = f2bf(ema_one(e, w, o));
+        uint32_t f, t;
+        rc_fragment_positions((uint32_t)i, f, t);
+        net.w16[f] = net.wT16[t] = f2bf(w);
+        net.wE16[f] = f2bf(ema_one(e, w, o));
         net.wE[i] = e;
     }
     if(i < entries)
@@ -426,10 +517,10 @@ __global__ __launch_bounds__(256) void k_rc_adam(DNrcNet net, DNrcAdam o, size_t
         reinterpret_cast<float2*>(net.tabM)[i] = m;
         reinterpret_cast<float2*>(net.tabV)[i] = v;
         reinterpret_cast<float2*>(net.tabGrad)[i] = make_float2(0.0f, 0.0f);
-        net.tab16[i] = (uint32_t)f2bf(w.x) | ((uint32_t)f2bf(w.y) << 16);
+        net.tab16[i] = f2bf2(w.x, w.y);
         const float ex = ema_one(e.x, w.x, o), ey = ema_one(e.y, w.y, o);
         reinterpret_cast<float2*>(net.tabE)[i] = e;
-        net.tabE16[i] = (uint32_t)f2bf(ex) | ((uint32_t)f2bf(ey) << 16);
+        net.tabE16[i] = f2bf2(ex, ey);
     }
 }
 
@@ -687,20 +778,21 @@ inline uint32_t blocks_for(size_t threads, uint32_t cap = 0x7FFFFFFFu)
 
 }  // namespace
 
-int dn_rc_encode(const DNrcNet& net, const float* samples, uint32_t n, uint16_t* x0, hipStream_t stream)
+namespace {
+void launch_encode(const DNrcNet& net, const float* samples, uint32_t n, uint32_t* x0, hipStream_t stream)
 {
-    if(n == 0) return 0;
-    hipLaunchKernelGGL(k_rc_encode, dim3(blocks_for((size_t)n * 16u)), dim3(256), 0, stream, net, samples, n, x0);
-    return (int)hipGetLastError();
+    hipLaunchKernelGGL(k_rc_encode, dim3(8u * blocks_for(n)), dim3(256), 0, stream, net, samples, n, x0);
 }
+}  // namespace
 
-int dn_rc_forward(const DNrcNet& net, const uint16_t* x0, const float* samples, uint32_t n, float* pred,
-                  hipStream_t stream)
+int dn_rc_predict(const DNrcNet& net, const float* samples, uint32_t n, float* pred, hipStream_t stream)
 {
     if(n == 0 || (n & 15u)) return n ? (int)hipErrorInvalidValue : 0;
-    DNrcActs none = {};
-    hipLaunchKernelGGL(k_rc_mlp<false>, dim3(blocks_for((size_t)n / 16u * 64u, 1024)), dim3(256), 0, stream, net, x0,
-                       samples, n, 0.0f, pred, none);
+    // at most three blocks a CU: more of them evict each other's table lines
+    // (10^6 rows, 2^19 entries: 181 us; 188 at 1024 blocks, 190 at 1536), fewer
+    // leave small tables waiting (2^14 entries: 120 us; 132 at 512 blocks)
+    hipLaunchKernelGGL(k_rc_predict, dim3(blocks_for((size_t)n * 4u, 768)), dim3(256), 0, stream, net, samples, n,
+                       pred);
     return (int)hipGetLastError();
 }
 
@@ -709,11 +801,11 @@ int dn_rc_train(const DNrcNet& net, const float* samples, uint32_t n, const DNrc
 {
     if(n == 0 || (n & 15u)) return n ? (int)hipErrorInvalidValue : 0;
     const uint32_t tiles = n / 16u;
-    hipLaunchKernelGGL(k_rc_encode, dim3(blocks_for((size_t)n * 16u)), dim3(256), 0, stream, net, samples, n, a.x0);
+    launch_encode(net, samples, n, a.x0, stream);
     // at most 512 blocks (4 tiles per wave at 2^17 samples): 83 us per 2^17 samples against 92 at
     // 1024 blocks, 98 at 256 and 82 at 768
-    hipLaunchKernelGGL(k_rc_mlp<true>, dim3(blocks_for((size_t)tiles * 64u, 512)), dim3(256), 0, stream, net,
-                       (const uint16_t*)a.x0, samples, n, 1.0f / (float)n, (float*)nullptr, a);
+    hipLaunchKernelGGL(k_rc_mlp, dim3(blocks_for((size_t)tiles * 64u, 512)), dim3(256), 0, stream, net, samples, n,
+                       1.0f / (float)n, a);
     // The weight gradients (MFMA and LDS bound) and the table gradients (bound
     // by their atomics) read the same activations and write disjoint buffers:
     // with a side stream they run side by side.
@@ -780,57 +872,4 @@ int dn_accumulate_f64(const float* src, double* dst, size_t n, hipStream_t strea
     if(n == 0) return 0;
     hipLaunchKernelGGL(k_accumulate_f64, dim3(blocks_for(n, 4096)), dim3(256), 0, stream, src, dst, n);
     return (int)hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Allocation-free prediction (DNX_rc_predict_samples_noalloc). The encoded
-// input rows that DNX_rc_predict_samples keeps in a query buffer grown with
-// hipMalloc live here in `scratch`, a fixed array that every device holds in
-// its own memory for the life of the process: DNX_RC_NOALLOC_MAX_SAMPLES rows
-// of RC_IN bf16 values (24 MiB). k_rc_encode writes every column of the rows
-// it is given and k_rc_mlp reads only those, so nothing needs clearing between
-// calls. In host code `scratch` names a host-side stand-in, not device memory:
-// kernels get the address that hipGetSymbolAddress gives for each device.
-static_assert(DNX_RC_NOALLOC_MAX_SAMPLES % 16u == 0u, "whole 16-sample tiles");
-static __device__ __align__(256) uint16_t scratch[(size_t)DNX_RC_NOALLOC_MAX_SAMPLES * RC_IN];
-
-namespace {
-std::mutex g_scratchLock;
-std::vector<uint16_t*> g_scratchAddr;     // per device: scratch's device address
-}  // namespace
-
-bool dn_noalloc_init()
-{
-    int count = 0, current = 0;
-    if(hipGetDeviceCount(&count) != hipSuccess || count < 1 || hipGetDevice(&current) != hipSuccess) return false;
-    std::lock_guard<std::mutex> lock(g_scratchLock);
-    if(g_scratchAddr.size() < (size_t)count) g_scratchAddr.resize((size_t)count, nullptr);
-    bool ok = true;
-    for(int d = 0; d < count; d++)
-    {
-        if(g_scratchAddr[d]) continue;                       // once per device
-        void* p = nullptr;
-        if(hipSetDevice(d) != hipSuccess || hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p)
-        {
-            ok = false;
-            continue;
-        }
-        g_scratchAddr[d] = static_cast<uint16_t*>(p);
-    }
-    if(hipSetDevice(current) != hipSuccess) ok = false;
-    return ok;
-}
-
-int dn_rc_predict_noalloc(const DNrcNet& net, int device, const float* samples, uint32_t n, float* pred,
-                          hipStream_t stream)
-{
-    if(n == 0 || (n & 15u) || n > DNX_RC_NOALLOC_MAX_SAMPLES) return (int)hipErrorInvalidValue;
-    uint16_t* x0 = nullptr;
-    {
-        std::lock_guard<std::mutex> lock(g_scratchLock);
-        if(device >= 0 && (size_t)device < g_scratchAddr.size()) x0 = g_scratchAddr[device];
-    }
-    if(!x0) return (int)hipErrorNotInitialized;
-    const int e = dn_rc_encode(net, samples, n, x0, stream);
-    return e ? e : dn_rc_forward(net, x0, samples, n, pred, stream);
 }

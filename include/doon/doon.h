@@ -473,11 +473,9 @@ bool DNX_rc_predict_samples(DNXradianceCache* rc, const float* samples, uint32_t
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): DNX_rc_predict_samples with the same inputs and outputs
  * and the same results, but calling no hipMalloc, hipFree or allocating
- * routine. Its encoded input rows live in a fixed per-device array of
- * DNX_RC_NOALLOC_MAX_SAMPLES rows (24 MiB, held by each device until the
- * process ends), set up by DN_init: n above that maximum is rejected (false,
- * ERROR message). Every call on a device shares that array, so calls that
- * overlap on one device (other streams, other threads) race. */
+ * routine. Rows are encoded inside the prediction kernel, so calls share no
+ * scratch memory and may overlap. At most DNX_RC_NOALLOC_MAX_SAMPLES rows, after
+ * DN_init: otherwise the call is rejected (false, ERROR message). */
 #define DNX_RC_NOALLOC_MAX_SAMPLES 262144u
 bool DNX_rc_predict_samples_noalloc(DNXradianceCache* rc, const float* samples, uint32_t n,
                                     float* out /* device float4 */);

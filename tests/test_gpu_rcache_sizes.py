@@ -1,0 +1,62 @@
+"""Radiance cache kernels at the sizes where their splits can go wrong: one
+16-row tile, a last wave without a tile, more tiles than resident waves, and
+tables whose levels are all hashed, dense and hashed in the same wave step, or
+mostly dense."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from doonengine_amd import scenes
+from doonengine_amd._hip import DeviceBuffer
+from doonengine_amd.volume import RadianceCache, Volume, rc_pack_weights
+from oracle import radiance_cache as orc
+
+pytestmark = pytest.mark.gpu
+
+EXTENT = 128.0
+
+
+@pytest.fixture(scope="module")
+def volume(gpu):
+    sc = scenes.config_small()
+    with Volume(sc.map_size, min_chunks=64) as vol:
+        yield vol
+
+
+def make_rows(rng, n):
+    s = np.zeros((n, 16), np.float32)
+    s[:, 0:3] = rng.uniform(-2.0, EXTENT + 2.0, (n, 3))        # past the extent on both sides
+    s[0, 0:3] = (0.0, EXTENT, 0.5 * EXTENT)
+    nrm = rng.normal(size=(n, 3))
+    s[:, 3:6] = nrm / np.linalg.norm(nrm, axis=1, keepdims=True)
+    s[:, 6:9] = rng.uniform(0.1, 0.9, (n, 3))
+    s[:, 9:12] = rng.uniform(0.0, 1.0, (n, 3))
+    s[:, 12] = 1.0
+    s[:, 13:16] = rng.uniform(0.0, 0.5, (n, 3))
+    return s
+
+
+@pytest.mark.parametrize("log2,n", [(10, 16), (14, 48), (15, 1040), (17, 4096 + 16), (19, 49152 + 80)])
+def test_a_batch_predicts_what_its_tiles_do(volume, log2, n):
+    """A row's prediction does not depend on the batch it comes in: 16-row calls
+    (whose outputs the oracle test checks) give the batch's bits."""
+    rng = np.random.default_rng(log2 * 1000 + n)
+    cfg = orc.Config(log2_table=log2, extent=EXTENT)
+    mats, table = orc.init_params(cfg, seed=9)
+    table = rng.normal(0, 0.1, table.shape).astype(np.float32)
+    rows = make_rows(rng, n)
+    rc = RadianceCache(volume, log2Table=log2, extent=EXTENT, samplesPerFrame=16)
+    try:
+        rc.set_params(rc_pack_weights(mats), table.reshape(-1))
+        out, one = DeviceBuffer(n * 16), DeviceBuffer(16 * 16)
+        rc.predict_samples(DeviceBuffer.from_array(rows), n, out)
+        volume.synchronize()
+        y = out.download(np.float32, (n, 4))
+        assert np.all(y[:, 3] == 1.0) and np.all(np.isfinite(y)) and np.abs(y[:, :3] - rows[:, 13:16]).max() > 0.0
+        for t in sorted({0, 1 % (n // 16), n // 32, n // 16 - 2 if n > 16 else 0, n // 16 - 1}):
+            rc.predict_samples(DeviceBuffer.from_array(rows[16 * t:16 * t + 16]), 16, one)
+            volume.synchronize()
+            assert np.array_equal(one.download(np.uint32, (16, 4)), y[16 * t:16 * t + 16].view(np.uint32)), t
+    finally:
+        rc.close()
