@@ -81,8 +81,20 @@ struct DNrcActs {
     uint16_t* hT[3];               // [tile][64][16]
     uint16_t* dzT[3];              // [tile][64][16]
     uint16_t* dyT;                 // [tile][16][16]
-    float* denc;                   // [samples][32]
+    float* denc;                   // [RC_LEVELS][samples][2] gradients of the encoded features
+    // Table gradients by bucket (rc_bucketed): positions over the extent, the
+    // records of every level, bucket and sorting block, those of every level and
+    // bucket, and per level 8 * samples record words in bucket order (16 * sample
+    // + which of its four corner rows meet the bucket).
+    float* unit;                   // [samples][4]
+    uint32_t* blockCount;          // [RC_LEVELS][RC_SORT_BLOCKS][RC_MAX_BUCKETS]
+    uint32_t* bucketCount;         // [RC_LEVELS][RC_MAX_BUCKETS]
+    uint32_t* records;
 };
+// A bucket: 2^12 consecutive table entries, whose gradients fill 64 KiB of LDS.
+enum { RC_BUCKET_LOG2 = 12, RC_MAX_BUCKETS = 128, RC_SORT_BLOCKS = 64, RC_BUCKETED_MAX = 1 << 24 };
+// Whether a step on n samples sorts its table gradients by bucket (n up to RC_BUCKETED_MAX).
+bool rc_bucketed(const DNrcNet& net, uint32_t n);
 struct DNrcAdam {
     float lr, beta1, beta2, eps;
     float bias1, bias2;            // 1 - beta^t

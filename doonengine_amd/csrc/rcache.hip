@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256) void k_rc_encode(DNrcNet net, const float* sam
     }
 }
 
-// Hash-table gradient, level-major: the waves running at a time work on one
+// Hash-table gradient of few samples, level-major: the waves running at a time work on one
 // level's gradient table (4 MiB at 2^19 entries), finest level first.
 // Device-scope FP32 atomics are served per cache line that one instruction
 // touches, not per lane (measured on MI355X: 64 lanes on 64 scattered lines
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_rc_table_grad(DNrcNet net, const float*
     const uint32_t s = (w % waves) * 16u + (lane >> 2);
     const uint32_t f = lane & 1u, xb = (lane >> 1) & 1u;
     if(s >= n) return;
-    const float d = denc[(size_t)s * RC_ENC + 2u * l + f];
+    const float d = denc[((size_t)l * n + s) * 2u + f];
     if(d == 0.0f) return;                                       // adding +-0 changes no sum
     float* gt = net.tabGrad + ((size_t)l << net.log2T) * 2u;
     const uint32_t N = net.res[l], mask = (1u << net.log2T) - 1u;
@@ -237,6 +237,277 @@ __global__ __launch_bounds__(256) void k_rc_table_grad(DNrcNet net, const float*
     {
         const uint32_t k = (j << 1) | xb;
         atomicAdd(gt + 2u * corner_index(N, dense, mask, cell, k) + f, corner_weight(cell, k) * d);
+    }
+}
+
+// Hash-table gradient of many samples, without global atomics on scattered
+// entries. Those are performed behind the L2s (giving each level to one XCD
+// changed nothing: 521 against 534 us per 2^17 samples of a terrain's surface at
+// 2^19 entries), so the table is cut into buckets of 2^12 entries, whose
+// gradients a block sums in LDS and adds to the table once. A sample's four
+// corner rows (y, z), of two x-neighbour corners each, are first sorted by
+// bucket: k_rc_bucket_count, then k_rc_bucket_place, which writes a word per
+// sample and bucket that it meets. A level that fits one bucket needs no records.
+// The sums are in FP64: LDS atomics on doubles take 22 cycles per wave here, on
+// floats 195 whatever the addresses (on 32-bit integers 9).
+
+__device__ __forceinline__ uint32_t level_buckets(const DNrcNet& net, uint32_t l)
+{
+    const uint32_t S = net.res[l] + 2u, T = 1u << net.log2T;
+    const uint32_t entries = ((net.denseMask >> l) & 1u) ? S * S * S : T;
+    return (entries + (1u << RC_BUCKET_LOG2) - 1u) >> RC_BUCKET_LOG2;
+}
+
+// The buckets that a sample's corners lie in, one of eight values per corner.
+struct SampleBuckets {
+    uint32_t b[8];
+    __device__ __forceinline__ SampleBuckets(uint32_t N, bool dense, uint32_t mask, const UnitPos& u)
+    {
+        const LevelCell c = level_cell(N, u);
+        #pragma unroll
+        for(uint32_t k = 0; k < 8u; k++) b[k] = corner_index(N, dense, mask, c, k) >> RC_BUCKET_LOG2;
+    }
+    // whether corner k is the first one in its bucket
+    __device__ __forceinline__ bool first(uint32_t k) const
+    {
+        bool is = true;
+        #pragma unroll
+        for(uint32_t i = 0; i < 8u; i++)
+            if(i < k && b[i] == b[k]) is = false;
+        return is;
+    }
+    // the rows with a corner in corner k's bucket
+    __device__ __forceinline__ uint32_t rows(uint32_t k) const
+    {
+        uint32_t m = 0u;
+        #pragma unroll
+        for(uint32_t i = 0; i < 8u; i++)
+            if(b[i] == b[k]) m |= 1u << (i >> 1);
+        return m;
+    }
+};
+
+// Sorting blocks take 4096 samples at a time, a thread four of them. Rows come in
+// runs of 32 neighbouring voxels. On a hashed level neighbouring lanes take
+// neighbouring rows: those with the same (y, z) stay neighbours in their bucket,
+// and k_rc_bucket_grad's gathers share cache lines. On a dense level they take
+// rows 32 apart: there lanes of one run would add to the same few entries.
+__device__ __forceinline__ uint32_t sort_sample(bool dense, uint32_t first, uint32_t t, uint32_t k)
+{
+    return first + (dense ? (t & 127u) * 32u + (t >> 7) + 8u * k : t + 1024u * k);
+}
+// First and last + 1 of a sorting block's samples, in whole 4096s.
+__device__ __forceinline__ uint32_t sort_span(uint32_t n)
+{
+    return ((n + 4095u) / 4096u + gridDim.x - 1u) / gridDim.x * 4096u;
+}
+
+// blockIdx.y: the level. The blocks of level 0 also write the unit positions,
+// with the divisions by the extent that the other kernels then need not make.
+__global__ __launch_bounds__(1024) void k_rc_bucket_count(DNrcNet net, const float* samples, uint32_t n, DNrcActs acts)
+{
+    __shared__ uint32_t hist[RC_MAX_BUCKETS];
+    const uint32_t l = blockIdx.y, t = threadIdx.x;
+    const uint32_t buckets = level_buckets(net, l);
+    if(buckets == 1u && l != 0u) return;
+    if(t < RC_MAX_BUCKETS) hist[t] = 0u;
+    __syncthreads();
+    const uint32_t N = net.res[l], mask = (1u << net.log2T) - 1u, span = sort_span(n);
+    const bool dense = (net.denseMask >> l) & 1u;
+    for(uint32_t f = blockIdx.x * span; f < blockIdx.x * span + span; f += 4096u)
+        for(uint32_t k = 0; k < 4u; k++)
+        {
+            const uint32_t s = sort_sample(dense, f, t, k);
+            if(s >= n) continue;
+            const UnitPos u = unit_pos(net, samples + (size_t)s * RC_SAMPLE);
+            if(l == 0u) reinterpret_cast<float4*>(acts.unit)[s] = make_float4(u.v[0], u.v[1], u.v[2], 0.0f);
+            if(buckets == 1u) continue;
+            const SampleBuckets sb(N, dense, mask, u);
+            #pragma unroll
+            for(uint32_t c = 0; c < 8u; c++)
+                if(sb.first(c)) atomicAdd(&hist[sb.b[c]], 1u);
+        }
+    __syncthreads();
+    if(buckets > 1u && t < RC_MAX_BUCKETS)
+        acts.blockCount[(l * RC_SORT_BLOCKS + blockIdx.x) * RC_MAX_BUCKETS + t] = hist[t];
+}
+
+__global__ __launch_bounds__(1024) void k_rc_bucket_place(DNrcNet net, uint32_t n, DNrcActs acts)
+{
+    __shared__ uint32_t next[RC_MAX_BUCKETS], firstHalf;
+    const uint32_t l = blockIdx.y, t = threadIdx.x;
+    const uint32_t buckets = level_buckets(net, l);
+    if(buckets == 1u) return;
+    // where this block's share of each bucket starts: the buckets in order, in
+    // each the blocks in order
+    uint32_t total = 0u, before = 0u, incl = 0u;
+    if(t < RC_MAX_BUCKETS)
+    {
+        const uint32_t* cnt = acts.blockCount + l * RC_SORT_BLOCKS * RC_MAX_BUCKETS + t;
+        for(uint32_t b = 0; b < gridDim.x; b++)
+        {
+            const uint32_t v = cnt[b * RC_MAX_BUCKETS];
+            if(b < blockIdx.x) before += v;
+            total += v;
+        }
+        if(blockIdx.x == 0u) acts.bucketCount[l * RC_MAX_BUCKETS + t] = total;
+        incl = total;
+        for(uint32_t off = 1u; off < 64u; off <<= 1)
+        {
+            const uint32_t v = __shfl_up(incl, off, 64);
+            if((t & 63u) >= off) incl += v;
+        }
+        if(t == 63u) firstHalf = incl;
+    }
+    __syncthreads();
+    if(t < RC_MAX_BUCKETS) next[t] = incl - total + before + (t >= 64u ? firstHalf : 0u);
+    __syncthreads();
+    const uint32_t N = net.res[l], mask = (1u << net.log2T) - 1u, span = sort_span(n);
+    const bool dense = (net.denseMask >> l) & 1u;
+    uint32_t* rec = acts.records + (size_t)l * 8u * n;
+    for(uint32_t f = blockIdx.x * span; f < blockIdx.x * span + span; f += 4096u)
+        for(uint32_t k = 0; k < 4u; k++)
+        {
+            const uint32_t s = sort_sample(dense, f, t, k);
+            if(s >= n) continue;
+            const float4 p = reinterpret_cast<const float4*>(acts.unit)[s];
+            const SampleBuckets sb(N, dense, mask, UnitPos{{p.x, p.y, p.z}});
+            #pragma unroll
+            for(uint32_t c = 0; c < 8u; c++)
+                if(sb.first(c)) rec[atomicAdd(&next[sb.b[c]], 1u)] = s * 16u + sb.rows(c);
+        }
+}
+
+// Sums one slice of a bucket in LDS. Blocks take the slices of all buckets in
+// turn; a bucket of one slice is added to the table by plain loads and stores,
+// one of several by atomics (consecutive entries: 16 to a cache line). Slices of
+// hashed levels are longer: their records hold one row each, mostly, those of
+// dense levels up to four.
+__device__ __forceinline__ uint32_t slice_records(bool dense) { return dense ? 2048u : 5120u; }
+
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8)))
+void k_rc_bucket_grad(DNrcNet net, uint32_t n, DNrcActs acts)
+{
+    __shared__ __align__(16) double acc[2u << RC_BUCKET_LOG2];
+    __shared__ uint32_t waveSums[16];
+    __shared__ uint32_t item[5];                    // level, bucket, first record, records, slices of the bucket
+    static_assert(RC_LEVELS == 16 && RC_MAX_BUCKETS == 128, "a wave per level, two buckets per thread");
+    const uint32_t t = threadIdx.x, lane = t & 63u, tl = t >> 6;
+    // this thread's two buckets: their records, and the slices of them and of all earlier ones
+    const uint32_t tn = level_buckets(net, tl), tslice = slice_records((net.denseMask >> tl) & 1u);
+    uint32_t cnt[2], slices[2];
+    for(uint32_t k = 0; k < 2u; k++)
+    {
+        const uint32_t b = 2u * lane + k;
+        cnt[k] = b >= tn ? 0u : (tn == 1u ? n : acts.bucketCount[tl * RC_MAX_BUCKETS + b]);
+        slices[k] = (cnt[k] + tslice - 1u) / tslice;
+    }
+    uint32_t start = cnt[0] + cnt[1], before = slices[0] + slices[1];
+    for(uint32_t off = 1u; off < 64u; off <<= 1)
+    {
+        const uint32_t a = __shfl_up(start, off, 64), b = __shfl_up(before, off, 64);
+        if(lane >= off) { start += a; before += b; }
+    }
+    if(lane == 63u) waveSums[tl] = before;
+    __syncthreads();
+    start -= cnt[0] + cnt[1];
+    before -= slices[0] + slices[1];
+    uint32_t total = 0u;
+    for(uint32_t w = 0; w < 16u; w++)
+    {
+        if(w == tl) before += total;
+        total += waveSums[w];
+    }
+    const uint32_t mask = (1u << net.log2T) - 1u;
+    const uint32_t sums = min(2u << RC_BUCKET_LOG2, 2u << net.log2T);
+    for(uint32_t it = blockIdx.x; it < total; it += gridDim.x)
+    {
+        for(uint32_t k = 0; k < 2u; k++)
+        {
+            const uint32_t at = before + (k ? slices[0] : 0u);
+            if(it < at || it >= at + slices[k]) continue;
+            const uint32_t o = (it - at) * tslice;
+            item[0] = tl; item[1] = 2u * lane + k; item[2] = start + (k ? cnt[0] : 0u) + o;
+            item[3] = min(tslice, cnt[k] - o); item[4] = slices[k];
+        }
+        for(uint32_t i = t; i < sums / 2u; i += 1024u) reinterpret_cast<double2*>(acc)[i] = make_double2(0.0, 0.0);
+        __syncthreads();
+        const uint32_t l = item[0], bucket = item[1], first = item[2], count = item[3], parts = item[4];
+        const uint32_t N = net.res[l], lo = bucket << RC_BUCKET_LOG2;
+        const bool dense = (net.denseMask >> l) & 1u, whole = level_buckets(net, l) == 1u;
+        const uint32_t* rec = acts.records + (size_t)l * 8u * n + first;
+        const float2* denc = reinterpret_cast<const float2*>(acts.denc) + (size_t)l * n;
+        // two records at a time, so that a wave waits for records and then for
+        // their samples once per two
+        const uint32_t whole32 = (count + 31u) / 32u;               // runs of 32 samples in a slice without records
+        for(uint32_t r0 = t; r0 < (whole ? whole32 * 32u : count); r0 += 2048u)
+        {
+            uint32_t s[2], rows[2];
+            float2 d[2];
+            float4 p[2];
+            #pragma unroll
+            for(uint32_t k = 0; k < 2u; k++)
+            {
+                const uint32_t r = r0 + 1024u * k;
+                s[k] = n;
+                if(whole)
+                {
+                    if(r < whole32 * 32u) s[k] = first + (r % whole32) * 32u + r / whole32;
+                    rows[k] = 15u;
+                }
+                else if(r < count)
+                {
+                    const uint32_t w = rec[r];
+                    s[k] = w >> 4;
+                    rows[k] = w & 15u;
+                }
+            }
+            #pragma unroll
+            for(uint32_t k = 0; k < 2u; k++)
+            {
+                d[k] = make_float2(0.0f, 0.0f);
+                if(s[k] >= n) continue;
+                d[k] = denc[s[k]];
+                p[k] = reinterpret_cast<const float4*>(acts.unit)[s[k]];
+            }
+            #pragma unroll
+            for(uint32_t k = 0; k < 2u; k++)
+            {
+                if(d[k].x == 0.0f && d[k].y == 0.0f) continue;     // adding +-0 changes no sum
+                const LevelCell c = level_cell(N, UnitPos{{p[k].x, p[k].y, p[k].z}});
+                for(uint32_t m = rows[k]; m; m &= m - 1u)
+                {
+                    const uint32_t j = (uint32_t)__builtin_ctz(m);
+                    for(uint32_t x = 0; x < 2u; x++)
+                    {
+                        const uint32_t i = corner_index(N, dense, mask, c, 2u * j + x);
+                        if((i >> RC_BUCKET_LOG2) != bucket) continue;
+                        const float w = corner_weight(c, 2u * j + x);
+                        double* a = acc + 2u * (i - lo);
+                        atomicAdd(a, (double)(w * d[k].x));
+                        atomicAdd(a + 1, (double)(w * d[k].y));
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        float* g = net.tabGrad + (((size_t)l << net.log2T) + lo) * 2u;
+        if(parts == 1u)
+            for(uint32_t i = t; i < sums / 2u; i += 1024u)
+            {
+                const double2 v = reinterpret_cast<const double2*>(acc)[i];
+                if(v.x == 0.0 && v.y == 0.0) continue;
+                float2 o = reinterpret_cast<float2*>(g)[i];
+                o.x += (float)v.x; o.y += (float)v.y;
+                reinterpret_cast<float2*>(g)[i] = o;
+            }
+        else
+            for(uint32_t i = t; i < sums; i += 1024u)
+            {
+                const float v = (float)acc[i];
+                if(v != 0.0f) atomicAdd(g + i, v);
+            }
+        __syncthreads();
     }
 }
 
@@ -417,8 +688,10 @@ __global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const float* sample
         {
             f32x4 d = mfma32(a_frag32(WT + RC_OFF_W0 + mb * 1024u, lane), dz[0], dz[1], zero);
             d = mfma32(a_frag32(WT + RC_OFF_W0 + mb * 1024u + 512u, lane), dz[2], dz[3], d);
-            reinterpret_cast<float4*>(acts.denc + (size_t)sm * RC_ENC + mb * 16u + 4u * q)[0] =
-                make_float4(d[0], d[1], d[2], d[3]);
+            // features 16 mb + 4 q + 0..3: levels 8 mb + 2 q and the next
+            float2* g = reinterpret_cast<float2*>(acts.denc) + (size_t)(8u * mb + 2u * q) * n + sm;
+            g[0] = make_float2(d[0], d[1]);
+            g[n] = make_float2(d[2], d[3]);
         }
     }
 }
@@ -778,13 +1051,6 @@ inline uint32_t blocks_for(size_t threads, uint32_t cap = 0x7FFFFFFFu)
 
 }  // namespace
 
-namespace {
-void launch_encode(const DNrcNet& net, const float* samples, uint32_t n, uint32_t* x0, hipStream_t stream)
-{
-    hipLaunchKernelGGL(k_rc_encode, dim3(8u * blocks_for(n)), dim3(256), 0, stream, net, samples, n, x0);
-}
-}  // namespace
-
 int dn_rc_predict(const DNrcNet& net, const float* samples, uint32_t n, float* pred, hipStream_t stream)
 {
     if(n == 0 || (n & 15u)) return n ? (int)hipErrorInvalidValue : 0;
@@ -796,12 +1062,29 @@ int dn_rc_predict(const DNrcNet& net, const float* samples, uint32_t n, float* p
     return (int)hipGetLastError();
 }
 
+// Below some 10^4 rows the three sorted launches cost more than the atomics of
+// the one (8192 rows, 2^14 / 2^19 entries: 81 / 77 us a step against 73 / 73;
+// 16384: 102 / 95 against 114 / 113; 131072: 212 / 217 against 603 / 588). Tables
+// above 2^19 entries would need more buckets than a level's scan holds.
+bool rc_bucketed(const DNrcNet& net, uint32_t n)
+{
+    return (1u << net.log2T) <= (uint32_t)RC_MAX_BUCKETS << RC_BUCKET_LOG2 && n >= 12288u && n <= RC_BUCKETED_MAX;
+}
+
 int dn_rc_train(const DNrcNet& net, const float* samples, uint32_t n, const DNrcActs& a, hipStream_t stream,
                 const DNrcSide* side)
 {
     if(n == 0 || (n & 15u)) return n ? (int)hipErrorInvalidValue : 0;
     const uint32_t tiles = n / 16u;
-    launch_encode(net, samples, n, a.x0, stream);
+    const bool bucketed = rc_bucketed(net, n);
+    hipLaunchKernelGGL(k_rc_encode, dim3(8u * blocks_for(n)), dim3(256), 0, stream, net, samples, n, a.x0);
+    if(bucketed)
+    {
+        const uint32_t chunks = (n + 4095u) / 4096u;
+        const dim3 grid(chunks < RC_SORT_BLOCKS ? chunks : (uint32_t)RC_SORT_BLOCKS, RC_LEVELS);
+        hipLaunchKernelGGL(k_rc_bucket_count, grid, dim3(1024), 0, stream, net, samples, n, a);
+        hipLaunchKernelGGL(k_rc_bucket_place, grid, dim3(1024), 0, stream, net, n, a);
+    }
     // at most 512 blocks (4 tiles per wave at 2^17 samples): 83 us per 2^17 samples against 92 at
     // 1024 blocks, 98 at 256 and 82 at 768
     hipLaunchKernelGGL(k_rc_mlp, dim3(blocks_for((size_t)tiles * 64u, 512)), dim3(256), 0, stream, net, samples, n,
@@ -820,8 +1103,25 @@ int dn_rc_train(const DNrcNet& net, const float* samples, uint32_t n, const DNrc
         ws = side->stream;
     }
     hipLaunchKernelGGL(k_rc_wgrad, dim3(wb), dim3(256), 0, ws, net, tiles, a);
-    // one wave per 16 samples and level
-    hipLaunchKernelGGL(k_rc_table_grad, dim3(blocks_for((size_t)RC_LEVELS * ((n + 15u) / 16u) * 64u)), dim3(256), 0,
+    if(bucketed)
+    {
+        // blocks take several slices where there are more than two per CU (all can be
+        // resident at once, and each counts the slices only once: 80 us per 2^17 samples
+        // against 101 with a block per slice)
+        uint32_t blocks = 0;
+        for(uint32_t l = 0; l < RC_LEVELS; l++)
+        {
+            const bool dense = (net.denseMask >> l) & 1u;
+            const uint32_t S = net.res[l] + 2u, entries = dense ? S * S * S : 1u << net.log2T;
+            const uint32_t buckets = (entries + (1u << RC_BUCKET_LOG2) - 1u) >> RC_BUCKET_LOG2;
+            const uint32_t records = dense || buckets == 1u ? n : 4u * n, slice = dense ? 2048u : 5120u;
+            blocks += buckets * ((records / buckets + slice - 1u) / slice);
+        }
+        hipLaunchKernelGGL(k_rc_bucket_grad, dim3(blocks < 512u ? blocks : 512u), dim3(1024), 0, stream, net, n, a);
+    }
+    else
+        // one wave per 16 samples and level
+        hipLaunchKernelGGL(k_rc_table_grad, dim3(blocks_for((size_t)RC_LEVELS * ((n + 15u) / 16u) * 64u)), dim3(256), 0,
                        stream, net, samples, n, (const float*)a.denc);
     if(side && (hipEventRecord(side->join, side->stream) != hipSuccess ||
                 hipStreamWaitEvent(stream, side->join, 0) != hipSuccess))

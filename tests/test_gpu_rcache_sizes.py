@@ -60,3 +60,35 @@ def test_a_batch_predicts_what_its_tiles_do(volume, log2, n):
             assert np.array_equal(one.download(np.uint32, (16, 4)), y[16 * t:16 * t + 16].view(np.uint32)), t
     finally:
         rc.close()
+
+
+@pytest.mark.parametrize("log2,n,narrow", [(8, 4096, False), (13, 4112, False), (14, 20000, False), (16, 4096, True),
+                                           (8, 12288, False), (13, 12304, False), (16, 16400, True),
+                                           (19, 32784, False), (19, 65536, True)])
+def test_many_rows_gradients_match_oracle(volume, log2, n, narrow):
+    """Table gradients sorted by bucket: tables smaller than a bucket, levels of
+    one and of many buckets, and (narrow: all rows within a few cells) buckets of
+    several slices. Relative Frobenius error as for the small batches."""
+    rng = np.random.default_rng(log2 * 1000 + n)
+    cfg = orc.Config(log2_table=log2, extent=EXTENT)
+    mats, table = orc.init_params(cfg, seed=3)
+    table = rng.normal(0, 0.05, table.shape).astype(np.float32)
+    rows = make_rows(rng, n)
+    if narrow:
+        rows[:, 0:3] = rng.uniform(40.0, 44.0, (n, 3))
+    rows[:, 13:16] = 0.0
+    rc = RadianceCache(volume, log2Table=log2, extent=EXTENT, samplesPerFrame=16)
+    try:
+        rc.set_params(rc_pack_weights(mats), table.reshape(-1))
+        rc.train_samples(DeviceBuffer.from_array(rows), n, step=False)
+        _, _, _, tg = rc.get_params()
+        tg = tg.reshape(table.shape).astype(np.float64)
+        rc.train_samples(DeviceBuffer.from_array(rows), n, step=False)
+        _, _, _, twice = rc.get_params()
+    finally:
+        rc.close()
+    pos = np.clip(rows[:, 0:3], 0.0, EXTENT)
+    ref = orc.forward_backward(cfg, mats, table, pos, rows[:, 3:6], rows[:, 6:9], rows[:, 9:12], bf16_ops=True)
+    d = ref["dtable"]
+    assert np.linalg.norm(tg - d) / np.linalg.norm(d) < 5e-3
+    assert np.linalg.norm(twice.reshape(table.shape) - 2.0 * tg) / np.linalg.norm(tg) < 1e-5      # calls add up
