@@ -127,22 +127,27 @@ __device__ __forceinline__ uint32_t select_bit32(uint32_t m, uint32_t k)
 // get_voxel_position's select (voxelShared.comp:172-224): the bit index of the
 // voxNum-th (from 0) stored voxel of a chunk, or -1 past the last one. `mask`
 // is a chunk record's 16-word mask (16-byte aligned): its four 16-byte pieces
-// are loaded at once, then the word holding the bit is found by popcounts.
+// are loaded at once and the word holding the bit is found by popcounts, by
+// selects only. The bit is searched for once, in that word: a search under a
+// branch per word runs for each word that any lane of the wave is in.
 __device__ __forceinline__ int32_t select_in(const uint32_t* mask, uint32_t voxNum)
 {
     const uint4* q = reinterpret_cast<const uint4*>(mask);
     const uint4 a = q[0], b = q[1], c4 = q[2], d = q[3];
     const uint32_t w[16] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c4.x, c4.y, c4.z, c4.w, d.x, d.y, d.z, d.w};
-    uint32_t count = 0;
-    int32_t result = -1;
+    uint32_t count = 0, word = 0, before = 0, at = 16;
     #pragma unroll
     for(uint32_t i = 0; i < 16; i++)
     {
-        const uint32_t bc = (uint32_t)__builtin_popcount(w[i]);
-        if(result < 0 && count + bc > voxNum) result = (int32_t)(i * 32u + select_bit32(w[i], voxNum - count));
-        count += bc;
+        const uint32_t next = count + (uint32_t)__builtin_popcount(w[i]);
+        const bool here = count <= voxNum && voxNum < next;
+        word = here ? w[i] : word;
+        before = here ? count : before;
+        at = here ? i : at;
+        count = next;
     }
-    return result;
+    const uint32_t bit = select_bit32(word, voxNum - before);
+    return at < 16u ? (int32_t)(at * 32u + bit) : -1;
 }
 
 // ---------------------------------------------------------------------------
@@ -254,27 +259,25 @@ __device__ __forceinline__ bool occ_bit(const uint32_t* bits, uint32_t idx)
     return (bits[idx >> 5] >> (idx & 31u)) & 1u;
 }
 
-// rank_in over a mask held in an LDS row (same arithmetic)
-__device__ __forceinline__ uint32_t rank_row(const uint32_t* row, const uint32_t partial[3], uint32_t li)
+// get_voxel_index without the pool base (voxelShared.comp:150-169), over a mask
+// held in an LDS row: `tail` is the record's fifth 16-byte piece, whose first
+// three words are the rank prefix. Straight-line: the four words are read at once.
+__device__ __forceinline__ uint32_t rank_row(const uint32_t* row, uint4 tail, uint32_t li)
 {
-    uint32_t w = li >> 5, q = w >> 2, j = w & 3u;
-    uint32_t n = q == 0 ? 0u : (q == 1 ? partial[0] : (q == 2 ? partial[1] : partial[2]));
+    const uint32_t q = li >> 7, j = (li >> 5) & 3u, part = (1u << (li & 31u)) - 1u;
     const uint32_t* v = row + 4u * q;
-    uint32_t part = (1u << (li & 31u)) - 1u;
-    uint32_t b0 = j == 0 ? (v[0] & part) : v[0];
-    uint32_t b1 = j == 1 ? (v[1] & part) : (j > 1 ? v[1] : 0u);
-    uint32_t b2 = j == 2 ? (v[2] & part) : (j > 2 ? v[2] : 0u);
-    uint32_t b3 = j == 3 ? (v[3] & part) : 0u;
-    return n + __builtin_popcount(b0) + __builtin_popcount(b1) + __builtin_popcount(b2) + __builtin_popcount(b3);
+    const uint32_t v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3];
+    const uint32_t m0 = j == 0u ? part : ~0u;
+    const uint32_t m1 = j == 1u ? part : (j > 1u ? ~0u : 0u);
+    const uint32_t m2 = j == 2u ? part : (j > 2u ? ~0u : 0u);
+    const uint32_t m3 = j == 3u ? part : 0u;
+    uint32_t n = q == 1u ? tail.x : 0u;
+    n = q == 2u ? tail.y : n;
+    n = q == 3u ? tail.z : n;
+    return n + __builtin_popcount(v0 & m0) + __builtin_popcount(v1 & m1) + __builtin_popcount(v2 & m2) +
+           __builtin_popcount(v3 & m3);
 }
 
-// step_chunk, voxelShared.comp:328-418. maxDepth is negative on every path here
-// (no raster compositing), so the depth test at :363 always passes.
-// LDSM: the chunk's occupancy mask goes to the lane's LDS row (c.maskRow) on
-// entry and each voxel trip reads one word of it, instead of selecting the
-// word out of 16 registers by a per-lane index. FINITE: the ray's delta is
-// finite on every axis, so iterate_dda_finite applies (never with refraction,
-// which changes the direction).
 // lastSideDist of voxelShared.comp: the side distances before the last step,
 // of which the walk only ever uses the minimum (the distance at which the ray
 // entered its current cell). The finite-delta walk keeps just that minimum
@@ -297,34 +300,39 @@ template <> struct LastSide<true> {
     __device__ __forceinline__ float minc() const { return t; }
 };
 
-template <bool REFRACT, bool LDSM = false, bool FINITE = false>
+// The chunk's occupancy mask in an LDS row: the row staged once for the whole
+// wave, or the lane's own, filled on entry. Each voxel trip then reads one word of
+// it, instead of selecting the word out of 16 registers by a per-lane index.
+__device__ __forceinline__ const uint32_t* stage_mask(const DNsceneView& s, const RayCtx& c, uint32_t mapIndex)
+{
+    if(mapIndex == c.sharedMap) return c.sharedRow;
+    const uint4* rq = reinterpret_cast<const uint4*>(s.chunks + mapIndex);
+    uint32_t* row = c.maskRow;
+    for(int k = 0; k < 4; k++)
+    {
+        const uint4 v = rq[k];
+        row[4 * k + 0] = v.x; row[4 * k + 1] = v.y; row[4 * k + 2] = v.z; row[4 * k + 3] = v.w;
+    }
+    return row;
+}
+
+__device__ __forceinline__ bool mask_row_bit(const uint32_t* row, uint32_t li)
+{
+    return (row[li >> 5] >> (li & 31u)) & 1u;
+}
+
+// step_chunk, voxelShared.comp:328-418. maxDepth is negative on every path here
+// (no raster compositing), so the depth test at :363 always passes. FINITE: the
+// ray's delta is finite on every axis, so iterate_dda_finite applies (never with
+// refraction, which changes the direction).
+template <bool REFRACT, bool FINITE>
 __device__ bool step_chunk(const DNsceneView& s, RayCtx& c, uint32_t mapIndex, f3& dir, f3& inv, f3& p,
                            bool ignoreFirst, f3& hitNormal, DVoxel& vox, f3& colorAdd, float& colorMult,
                            bool& refracted)
 {
     refracted = false;
-    const DNchunkRec* rec = s.chunks + mapIndex;
-    const uint4* rq = reinterpret_cast<const uint4*>(rec);
-    Mask512 m;
-    const uint32_t* mrow = c.maskRow;
-    if(LDSM)
-    {
-        if(mapIndex == c.sharedMap)
-            mrow = c.sharedRow;            // staged once for the whole wave
-        else
-        {
-            uint32_t* row = c.maskRow;
-            for(int k = 0; k < 4; k++)
-            {
-                uint4 v = rq[k];
-                row[4 * k + 0] = v.x; row[4 * k + 1] = v.y; row[4 * k + 2] = v.z; row[4 * k + 3] = v.w;
-            }
-        }
-    }
-    else
-    {
-        m.q[0] = rq[0]; m.q[1] = rq[1]; m.q[2] = rq[2]; m.q[3] = rq[3];
-    }
+    const uint4* rq = reinterpret_cast<const uint4*>(s.chunks + mapIndex);
+    const uint32_t* mrow = stage_mask(s, c, mapIndex);
     DDA d;
     init_dda(dir, inv, p, d);
     LastSide<FINITE> lsd;
@@ -333,12 +341,10 @@ __device__ bool step_chunk(const DNsceneView& s, RayCtx& c, uint32_t mapIndex, f
     {
         c.sVox++;
         uint32_t li = (uint32_t)(d.px + 8 * (d.py + 8 * d.pz));
-        const uint32_t bit = LDSM ? (mrow[li >> 5] >> (li & 31u)) & 1u : mask_bit(m, li);
-        if(bit && !ignoreFirst)
+        if(mask_row_bit(mrow, li) && !ignoreFirst)
         {
-            uint4 tail = rq[4];   // partial[0..2], voxelIndex
-            uint32_t partial[3] = {tail.x, tail.y, tail.z};
-            uint32_t idx = tail.w + (LDSM ? rank_row(mrow, partial, li) : rank_in(m, partial, li));
+            const uint4 tail = rq[4];   // partial[0..2], voxelIndex
+            uint32_t idx = tail.w + rank_row(mrow, tail, li);
             uint4 cw = s.voxels[idx];
             vox = decompress(cw);
             const DNmat& mat = s.mats[vox.material];
@@ -395,11 +401,53 @@ __device__ bool step_chunk(const DNsceneView& s, RayCtx& c, uint32_t mapIndex, f
     return false;
 }
 
-// step_map, voxelShared.comp:421-475
-template <bool REFRACT, bool LDSM = false, bool FINITE = false>
+// step_chunk where every stored voxel is opaque (DNsceneView::opaque): the first
+// stored voxel is the hit, whatever it holds, and no ray is ever inside one. The
+// loop then only walks: one exit test per trip, no look-up of voxels and
+// materials. In the general loop that look-up, three dependent loads and some 150
+// instructions, runs once for each trip at which some lane of the wave hits.
+// `li` receives the hit voxel's position in the chunk.
+template <bool FINITE>
+__device__ __forceinline__ bool step_chunk_opaque(const DNsceneView& s, RayCtx& c, uint32_t mapIndex, f3 dir, f3 inv,
+                                                  f3& p, bool ignoreFirst, f3& hitNormal, uint32_t& li)
+{
+    const uint32_t* mrow = stage_mask(s, c, mapIndex);
+    DDA d;
+    init_dda(dir, inv, p, d);
+    LastSide<FINITE> lsd;
+    if(!in_chunk_cell(d)) return false;
+    li = (uint32_t)(d.px + 8 * (d.py + 8 * d.pz));
+    bool stored = mask_row_bit(mrow, li) && !ignoreFirst, inside = true;
+    c.sVox++;
+    if(!stored)
+        do
+        {
+            lsd.set(d.side);
+            if(FINITE) iterate_dda_finite(d, hitNormal);
+            else iterate_dda(d, hitNormal);
+            inside = in_chunk_cell(d);
+            c.sVox++;
+            li = (uint32_t)(d.px + 8 * (d.py + 8 * d.pz)) & 511u;    // a cell outside reads some word of the row
+            stored = mask_row_bit(mrow, li);
+        } while(inside && !stored);
+    if(!inside)
+    {
+        c.sVox--;
+        return false;
+    }
+    p = p + dir * (lsd.minc() + DN_EPS);
+    return true;
+}
+
+// step_map, voxelShared.comp:421-475. LIGHT: a lighting ray, which does not refract
+// and ends once it can meet nothing more (below). OPAQUE: every stored voxel is
+// opaque. VOXEL: false leaves out what the ray hit (`vox` and c.hitIndex).
+template <bool LIGHT, bool OPAQUE, bool FINITE = false, bool VOXEL = true>
 __device__ bool step_map(const DNsceneView& s, RayCtx& c, f3& dir, f3 inv, f3& p, bool ignoreFirst, f3& hitNormal,
                          DVoxel& vox, f3& colorAdd, float& colorMult)
 {
+    static_assert(OPAQUE || VOXEL, "transparent voxels are looked up on the way");
+    constexpr bool REFRACT = !LIGHT && !OPAQUE;
     bool requested = false;
     colorAdd = splat(0.0f);
     colorMult = 1.0f;
@@ -408,28 +456,31 @@ __device__ bool step_map(const DNsceneView& s, RayCtx& c, f3& dir, f3 inv, f3& p
     init_dda(dir, inv, p, d);
     LastSide<FINITE> lsd;
     bool hit = false;
+    uint32_t idx = 0, li = 0;
     const int32_t X = (int32_t)s.mapX, Y = (int32_t)s.mapY, Z = (int32_t)s.mapZ;
     // a lighting ray that does not move down reads the column table of its
     // quadrant: the highest present tile over the columns it can still reach
-    const bool colRule = !REFRACT && s.colTop != nullptr && d.sy >= 0;
+    const bool colRule = LIGHT && s.colTop != nullptr && d.sy >= 0;
     const uint32_t colBase = ((d.sx > 0 ? 1u : 0u) + (d.sz > 0 ? 2u : 0u)) * s.mapX * s.mapZ;
     while(in_map_cell(d, (uint32_t)X, (uint32_t)Y, (uint32_t)Z))
     {
         c.sMap++;
         const int32_t colTop = colRule ? s.colTop[colBase + (uint32_t)d.px + s.mapX * (uint32_t)d.pz] : INT32_MAX;
-        uint32_t idx = (uint32_t)d.px + s.mapX * ((uint32_t)d.py + s.mapY * (uint32_t)d.pz);
+        idx = (uint32_t)d.px + s.mapX * ((uint32_t)d.py + s.mapY * (uint32_t)d.pz);
         if(occ_bit(s.occLoaded, idx))
         {
             s.lastUsed[idx] = 0u;          // a plain store: no read on the ray's path
             f3 upd = p + dir * (lsd.minc() - DN_EPS);
             f3 crp = (upd - mk((float)d.px, (float)d.py, (float)d.pz)) * 8.0f;
             crp = vclamp(crp, DN_EPS, 8.0f - DN_EPS);
-            bool refr;
-            if(step_chunk<REFRACT, LDSM, FINITE>(s, c, idx, dir, inv, crp, ignoreFirst, hitNormal, vox, colorAdd, colorMult,
-                                         refr))
+            bool refr = false;
+            if constexpr(OPAQUE) hit = step_chunk_opaque<FINITE>(s, c, idx, dir, inv, crp, ignoreFirst, hitNormal, li);
+            else
+                hit = step_chunk<REFRACT, FINITE>(s, c, idx, dir, inv, crp, ignoreFirst, hitNormal, vox, colorAdd,
+                                                  colorMult, refr);
+            if(hit)
             {
                 p = mk((float)d.px, (float)d.py, (float)d.pz) + crp * 0.125f;
-                hit = true;
                 break;
             }
             if(REFRACT && refr)
@@ -457,11 +508,19 @@ __device__ bool step_map(const DNsceneView& s, RayCtx& c, f3& dir, f3 inv, f3& p
         // still reach from the cell it just left (its y only grows and those
         // columns include all of its later ones). Only the trip counters
         // differ from the reference walk's; the oracle applies the same rules.
-        if(!REFRACT && ((d.sx > 0 ? d.px > s.presHi[0] : d.px < s.presLo[0]) ||
-                        (d.sy > 0 ? d.py > s.presHi[1] : d.py < s.presLo[1]) ||
-                        (d.sz > 0 ? d.pz > s.presHi[2] : d.pz < s.presLo[2]) || d.py > colTop))
+        if(LIGHT && ((d.sx > 0 ? d.px > s.presHi[0] : d.px < s.presLo[0]) ||
+                     (d.sy > 0 ? d.py > s.presHi[1] : d.py < s.presLo[1]) ||
+                     (d.sz > 0 ? d.pz > s.presHi[2] : d.pz < s.presLo[2]) || d.py > colTop))
             break;
     }
+    if constexpr(OPAQUE && VOXEL)
+        if(hit)                            // once per ray, all lanes of the wave that hit together
+        {
+            const uint4 tail = reinterpret_cast<const uint4*>(s.chunks + idx)[4];
+            const uint32_t* mrow = idx == c.sharedMap ? c.sharedRow : c.maskRow;
+            c.hitIndex = tail.w + rank_row(mrow, tail, li);
+            vox = decompress(s.voxels[c.hitIndex]);
+        }
     c.cRays++;
     c.cMap += c.sMap;
     c.cVox += c.sVox;

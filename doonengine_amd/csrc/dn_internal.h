@@ -42,6 +42,7 @@ struct DNsceneView {
     const DNmat* mats;           // 256
     uint32_t mapX, mapY, mapZ;
     uint32_t hasUnloaded;        // any tile in state 1/3: rays may request chunks
+    uint32_t opaque;             // every material that a voxel in the pool has held has opacity 1
     float sunStrength[3];
     float skyBot[3], skyTop[3];
     const uchar4* cube;          // sky cubemap: 6 faces (+X, -X, +Y, -Y, +Z, -Z) of cubeSize^2 RGBA8, or null
@@ -129,6 +130,7 @@ struct DNbatchParams {
     uint32_t numScenes;
     uint32_t unit;                 // requests per work unit, even
     uint32_t queues;               // 1 or 8
+    uint32_t opaque;               // every volume is (DNsceneView::opaque)
     uint32_t dry;                  // 1: compute only, no stores (autotuning)
     uint32_t* dryLastUsed;         // dry: where rays' lastUsed stores go instead (>= the largest volume's tiles)
     uint32_t* queueCounters;       // [queues] next unit of each queue

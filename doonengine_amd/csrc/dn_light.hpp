@@ -9,22 +9,25 @@ namespace {
 // voxelLighting.comp calls it, with the chunk masks in the lane's LDS row
 // (c.maskRow, set by every kernel that traces lighting rays). The nested
 // chunk-in-map loops are measured faster here than the single flattened loop.
+template <bool OPAQUE, bool VOXEL = true>
 __device__ __forceinline__ bool light_trace(const DNsceneView& s, RayCtx& c, f3 dir, f3 inv, f3& p, DVoxel& vox,
                                             f3& ca, float& cm)
 {
     f3 tn = splat(0.0f);
-    return step_map<false, true>(s, c, dir, inv, p, true, tn, vox, ca, cm);
+    return step_map<true, OPAQUE, false, VOXEL>(s, c, dir, inv, p, true, tn, vox, ca, cm);
 }
 
 // light_trace for the frame-uniform shadow directions (the same for every
 // voxel, so the test is uniform across the wave): the finite-delta walk when
-// no direction component is zero.
+// no direction component is zero. What the ray hit is not looked up where nothing
+// on its way can be transparent.
+template <bool OPAQUE>
 __device__ __forceinline__ bool light_trace_uniform(const DNsceneView& s, RayCtx& c, f3 dir, f3 inv, f3& p,
                                                     DVoxel& vox, f3& ca, float& cm)
 {
     f3 tn = splat(0.0f);
-    if(all_finite(inv)) return step_map<false, true, true>(s, c, dir, inv, p, true, tn, vox, ca, cm);
-    return step_map<false, true>(s, c, dir, inv, p, true, tn, vox, ca, cm);
+    if(all_finite(inv)) return step_map<true, OPAQUE, true, !OPAQUE>(s, c, dir, inv, p, true, tn, vox, ca, cm);
+    return step_map<true, OPAQUE, false, !OPAQUE>(s, c, dir, inv, p, true, tn, vox, ca, cm);
 }
 
 // The calling lane's row of a block's mask rows.
@@ -56,6 +59,7 @@ __device__ __forceinline__ f3 voxel_origin(const DNchunkRec* rec, int32_t sel, f
     return p + splat(0.0625f - DN_EPS) * normal;
 }
 
+template <bool OPAQUE>
 __device__ void shadow_ray(LCtx& L, f3 p, uint32_t sample, f3& color)
 {
     const DNlightParams& P = *L.P;
@@ -66,7 +70,7 @@ __device__ void shadow_ray(LCtx& L, f3 p, uint32_t sample, f3& color)
     {
         const float* r = L.firstSample ? P.firstShadow : P.shadowRays[sample];
         f3 pp = p;
-        if(!light_trace(*L.s, *L.c, ld3(r), ld3(r + 3), pp, hv, ca, cm))
+        if(!light_trace<OPAQUE, !OPAQUE>(*L.s, *L.c, ld3(r), ld3(r + 3), pp, hv, ca, cm))
             color = color + (L.sunStrength * cm + ca);
         return;
     }
@@ -87,12 +91,13 @@ __device__ void shadow_ray(LCtx& L, f3 p, uint32_t sample, f3& color)
     for(uint32_t k = 0; k < P.numDirectRays; k++)
     {
         f3 pp = p;
-        if(!light_trace_uniform(*L.s, *L.c, ld3(P.directRays[k]), ld3(P.directRays[k] + 3), pp, hv, ca, cm))
+        if(!light_trace_uniform<OPAQUE>(*L.s, *L.c, ld3(P.directRays[k]), ld3(P.directRays[k] + 3), pp, hv, ca, cm))
             acc = acc + (L.sunStrength * cm + ca);
     }
     color = color + acc / (float)P.numDirectRays;
 }
 
+template <bool OPAQUE>
 __device__ void specular_ray(LCtx& L, uint32_t thisMapIndex, f3 p, f3 dir, f3 albedo, uint32_t reflectType, f3& color)
 {
     const DNlightParams& P = *L.P;
@@ -103,7 +108,7 @@ __device__ void specular_ray(LCtx& L, uint32_t thisMapIndex, f3 p, f3 dir, f3 al
     for(uint32_t i = 0; i < P.specBounceLimit; i++)
     {
         f3 ca; float cm;
-        if(light_trace(s, *L.c, dir, vinv(dir), p, hv, ca, cm))
+        if(light_trace<OPAQUE>(s, *L.c, dir, vinv(dir), p, hv, ca, cm))
         {
             int32_t hx = (int32_t)p.x, hy = (int32_t)p.y, hz = (int32_t)p.z;
             uint32_t hitIdx = (uint32_t)hx + s.mapX * ((uint32_t)hy + s.mapY * (uint32_t)hz);
@@ -154,7 +159,7 @@ struct FrameRandom {
     __device__ f3 diffuse_dir(uint32_t sample, uint32_t i) const { return ld3(r->diffuseDir[sample][i]); }
 };
 
-template <typename RNG>
+template <bool OPAQUE, typename RNG>
 __device__ void diffuse_ray(LCtx& L, f3 normal, f3 p, const DVoxel& initial, uint32_t sample, f3& color,
                             const RNG& rng)
 {
@@ -179,7 +184,7 @@ __device__ void diffuse_ray(LCtx& L, f3 normal, f3 p, const DVoxel& initial, uin
         f3 ca;
         float cm;
         DVoxel nv = {};
-        bool hit = light_trace(s, *L.c, dir, vinv(dir), p, nv, ca, cm);
+        bool hit = light_trace<OPAQUE>(s, *L.c, dir, vinv(dir), p, nv, ca, cm);
         if(hit)
         {
             hv = nv;
@@ -208,6 +213,7 @@ __device__ void diffuse_ray(LCtx& L, f3 normal, f3 p, const DVoxel& initial, uin
 
 __device__ __forceinline__ uint32_t rne_u(float x) { return (uint32_t)rintf(x); }
 
+template <bool OPAQUE>
 __device__ void light_voxel(const DNlightParams& P, const DNsceneView& s, uint32_t r, uint32_t lane32, RayCtx& c,
                             uint32_t& lit, bool dry)
 {
@@ -249,7 +255,7 @@ __device__ void light_voxel(const DNlightParams& P, const DNsceneView& s, uint32
         for(uint32_t i = 0; i < P.numSpecRays; i++)
         {
             f3 sd = vnorm(refl * (float)mat.shininess + ld3(P.specPoints + 3 * i)) + DN_EPS;
-            specular_ray(L, mapIndex, p, sd, me.albedo, mat.reflectType, spec);
+            specular_ray<OPAQUE>(L, mapIndex, p, sd, me.albedo, mat.reflectType, spec);
         }
         spec = spec / (float)P.numSpecRays;
     }
@@ -260,8 +266,8 @@ __device__ void light_voxel(const DNlightParams& P, const DNsceneView& s, uint32
         for(uint32_t i = 0; i < P.numDiffuseSamples; i++)
         {
             diff = diff + ld3(P.ambient);
-            diffuse_ray(L, me.normal + DN_EPS, p, me, i, diff, rng);
-            shadow_ray(L, p, i, diff);
+            diffuse_ray<OPAQUE>(L, me.normal + DN_EPS, p, me, i, diff, rng);
+            shadow_ray<OPAQUE>(L, p, i, diff);
         }
         if(P.numDiffuseSamples) fresh = diff / (float)P.numDiffuseSamples;
         diff = (me.diffuse * indirect + diff) / (indirect + (float)P.numDiffuseSamples);

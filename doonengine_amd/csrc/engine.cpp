@@ -203,6 +203,7 @@ struct DNgpuVolume {
     DNmaterial lastMats[DN_MAX_MATERIALS];
     bool matsValid = false;
     bool anySpecular = false;
+    uint64_t usedMats[4] = {0, 0, 0, 0};   // materials of the voxels uploaded so far, one bit each
 
     bool timing = false;
     std::vector<Timer> pendingTimers;
@@ -384,7 +385,8 @@ void free_node(DNgpuVolume* g, uint32_t t)
 }
 
 // _DN_check_face_visible / _DN_chunk_to_gpu (voxel.c:1391-1461): per-chunk face
-// culling, occupancy mask, rank prefix, albedo linearisation.
+// culling, occupancy mask, rank prefix, albedo linearisation. `used`: the bits
+// of the stored voxels' materials are set.
 uint8_t g_linLUT[256];
 bool g_lutReady = false;
 
@@ -400,7 +402,7 @@ void build_lut()
     g_lutReady = true;
 }
 
-uint32_t chunk_to_gpu(const DNmaterial* mats, const DNchunk& ch, DNchunkRec& rec, uint4* vox)
+uint32_t chunk_to_gpu(const DNmaterial* mats, const DNchunk& ch, DNchunkRec& rec, uint4* vox, uint64_t used[4])
 {
     memset(&rec, 0, sizeof(rec));
     rec.pos[0] = ch.pos.x; rec.pos[1] = ch.pos.y; rec.pos[2] = ch.pos.z;
@@ -422,6 +424,8 @@ uint32_t chunk_to_gpu(const DNmaterial* mats, const DNchunk& ch, DNchunkRec& rec
              faceVisible(x, y - 1, z) || faceVisible(x, y, z + 1) || faceVisible(x, y, z - 1)))
             continue;
         rec.mask[index >> 5] |= 1u << (index & 31u);
+        const uint32_t mat = material_of(v.normal);
+        used[mat >> 6] |= 1ull << (mat & 63u);
         uint32_t a = v.albedo;
         uint32_t r = g_linLUT[(a >> 24) & 255u], gg = g_linLUT[(a >> 16) & 255u], b = g_linLUT[(a >> 8) & 255u];
         vox[n] = make_uint4(v.normal, (r << 24) | (gg << 16) | (b << 8), 0u, 0u);
@@ -643,6 +647,16 @@ bool upload_column_tops(DNvolume* vol)
     return ok;
 }
 
+// Whether no ray can meet a transparent voxel: every material that a voxel of the
+// pool has held since the volume was created has opacity exactly 1 now.
+bool all_opaque(const DNgpuVolume* g, const DNmaterial* mats)
+{
+    for(int k = 0; k < 4; k++)
+        for(uint64_t m = g->usedMats[k]; m; m &= m - 1)
+            if(mats[64 * k + __builtin_ctzll(m)].opacity != 1.0f) return false;
+    return true;
+}
+
 DNsceneView scene_view(DNvolume* vol)
 {
     DNgpuVolume* g = vol->gpu;
@@ -656,6 +670,7 @@ DNsceneView scene_view(DNvolume* vol)
     s.mats = g->dMats;
     s.mapX = vol->mapSize.x; s.mapY = vol->mapSize.y; s.mapZ = vol->mapSize.z;
     s.hasUnloaded = g->numUnloaded > 0 ? 1u : 0u;
+    s.opaque = g->matsValid && all_opaque(g, g->lastMats) ? 1u : 0u;
     s.sunStrength[0] = vol->sunStrength.x; s.sunStrength[1] = vol->sunStrength.y; s.sunStrength[2] = vol->sunStrength.z;
     s.skyBot[0] = vol->skyGradientBot.x; s.skyBot[1] = vol->skyGradientBot.y; s.skyBot[2] = vol->skyGradientBot.z;
     s.skyTop[0] = vol->skyGradientTop.x; s.skyTop[1] = vol->skyGradientTop.y; s.skyTop[2] = vol->skyGradientTop.z;
@@ -1104,12 +1119,15 @@ void stream_chunks(DNvolume* vol)
         const DNmaterial* mats = vol->materials;
         unsigned nth = std::min<unsigned>(8, std::max<unsigned>(1, std::thread::hardware_concurrency()));
         if(loads.size() < 64) nth = 1;
+        uint64_t used[8][4] = {};
         auto work = [&](unsigned w) {
+            uint64_t bits[4] = {0, 0, 0, 0};
             for(size_t i = w; i < loads.size(); i += nth)
             {
                 const DNchunk& ch = vol->chunks[vol->map[loads[i]].chunkIndex];
-                counts[i] = chunk_to_gpu(mats, ch, recs[i], &voxBuf[i * 512]);
+                counts[i] = chunk_to_gpu(mats, ch, recs[i], &voxBuf[i * 512], bits);
             }
+            memcpy(used[w], bits, sizeof(bits));
         };
         if(nth == 1) work(0);
         else
@@ -1118,6 +1136,8 @@ void stream_chunks(DNvolume* vol)
             for(unsigned w = 0; w < nth; w++) th.emplace_back(work, w);
             for(auto& x : th) x.join();
         }
+        for(unsigned w = 0; w < nth; w++)
+            for(int k = 0; k < 4; k++) g->usedMats[k] |= used[w][k];
     }
     size_t totalVox = 0;
     for(uint32_t n : counts) totalVox += n;
@@ -2769,6 +2789,7 @@ extern "C" void DNX_cast_rays(DNvolume* vol, uint32_t n, const float* origins, c
                               DNXrayHit* out)
 {
     DNgpuVolume* g = vol->gpu;
+    if(!upload_materials(vol)) return;
     DNrayParams p;
     p.scene = scene_view(vol);
     p.n = n;
@@ -2777,7 +2798,6 @@ extern "C" void DNX_cast_rays(DNvolume* vol, uint32_t n, const float* origins, c
     p.ignoreFirst = ignoreFirst ? 1u : 0u;
     p.out = out;
     p.counters = g->dCounters + 2 * CNT_SLOTS;
-    if(!upload_materials(vol)) return;
     Timer tm = timer_begin(g, TK_RAYS);
     int e = dn_launch_rays(p, g->stream);
     timer_end(g, tm);
@@ -2858,8 +2878,9 @@ struct DNXbatch {
     hipGraphExec_t exec[2] = {nullptr, nullptr};
     DNXbatchConfig execCfg[2];
     uint32_t execTiles[2] = {0, 0}, execReq[2] = {0, 0};
-    bool execDirect[2] = {false, false};
+    bool execDirect[2] = {false, false}, execOpaque[2] = {false, false};
     bool anyDirect = false;                           // some volume traces its direct rays ahead this frame
+    bool allOpaque = false;                           // no volume has transparent voxels this frame
     bool timing = true;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pending, spare;
     double ms = 0.0;
@@ -2904,6 +2925,7 @@ DNbatchParams batch_params(DNXbatch* b, bool dry)
     bp.numScenes = (uint32_t)b->vols.size();
     bp.unit = b->cfg.requestsPerUnit;
     bp.queues = b->queues;
+    bp.opaque = b->allOpaque ? 1u : 0u;
     bp.dry = dry ? 1u : 0u;
     bp.queueCounters = b->dQueueCounters;
     bp.directCounters = b->dQueueCounters + DN_BATCH_MAX_QUEUES;
@@ -2922,6 +2944,7 @@ bool batch_prepare(DNXbatch* b, DNlightParams* dst, int nds, int mds, float time
     maxTiles = 0;
     maxReq = 0;
     b->anyDirect = false;
+    b->allOpaque = true;
     for(size_t i = 0; i < b->vols.size(); i++)
     {
         DNvolume* vol = b->vols[i];
@@ -2935,6 +2958,7 @@ bool batch_prepare(DNXbatch* b, DNlightParams* dst, int nds, int mds, float time
             dst[i].directSlots = (uint32_t)std::min<size_t>(g->directCap, 0xFFFFFFFFu);
             b->anyDirect = true;
         }
+        b->allOpaque = b->allOpaque && dst[i].scene.opaque != 0u;
         maxTiles = std::max(maxTiles, vol->gpu->tiles);
         maxReq = std::max(maxReq, mr);
         // the batch stream waits for the work queued on the volume's stream (its
@@ -3044,7 +3068,7 @@ extern "C" bool DNX_batch_update_lighting(DNXbatch* b, int numDiffuseSamples, in
     const DNXbatchConfig& e = b->execCfg[s];
     bool stale = !b->exec[s] || e.requestsPerUnit != c.requestsPerUnit || e.blockThreads != c.blockThreads ||
                  e.blocksPerCU != c.blocksPerCU || e.xcdQueues != c.xcdQueues || b->execTiles[s] != maxTiles ||
-                 b->execReq[s] != maxReq || b->execDirect[s] != b->anyDirect;
+                 b->execReq[s] != maxReq || b->execDirect[s] != b->anyDirect || b->execOpaque[s] != b->allOpaque;
     if(stale)
     {
         if(b->exec[s]) { hipGraphExecDestroy(b->exec[s]); b->exec[s] = nullptr; }
@@ -3070,6 +3094,7 @@ extern "C" bool DNX_batch_update_lighting(DNXbatch* b, int numDiffuseSamples, in
         b->execTiles[s] = maxTiles;
         b->execReq[s] = maxReq;
         b->execDirect[s] = b->anyDirect;
+        b->execOpaque[s] = b->allOpaque;
     }
     std::pair<hipEvent_t, hipEvent_t> t(nullptr, nullptr);
     if(b->timing)

@@ -31,6 +31,7 @@ __device__ f3 voxel_color(const DNsceneView& s, uint32_t viewMode, DVoxel vox, f
 
 // One pixel's primary ray (voxelDraw.comp:24-147). The per-ray refraction state
 // starts afresh for every pixel, as the shader's per-invocation globals do.
+template <bool OPAQUE>
 __device__ __forceinline__ void draw_pixel(const DNdrawParams& P, const DNsceneView& s, RayCtx& c, uint32_t x,
                                            uint32_t y)
 {
@@ -66,7 +67,7 @@ __device__ __forceinline__ void draw_pixel(const DNdrawParams& P, const DNsceneV
         f3 nrm = vnorm(tr);
         DVoxel vox = {};
         f3 ca; float cm;
-        bool hit = step_map<true, true>(s, c, dir, inv, p, false, nrm, vox, ca, cm);
+        bool hit = step_map<false, OPAQUE>(s, c, dir, inv, p, false, nrm, vox, ca, cm);
         info.mapSteps = c.sMap; info.voxelSteps = c.sVox;
         if(hit)
         {
@@ -100,6 +101,7 @@ __device__ __forceinline__ void draw_pixel(const DNdrawParams& P, const DNsceneV
 #ifndef DN_DRAW_WAVES
 #define DN_DRAW_WAVES 4
 #endif
+template <bool OPAQUE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DN_DRAW_WAVES, DN_DRAW_WAVES)))
 void k_draw(DNdrawParams P)
 {
@@ -132,7 +134,7 @@ void k_draw(DNdrawParams P)
         if(x < P.width && y < P.height)
         {
             drawn++;
-            draw_pixel(P, sv, c, x, y);
+            draw_pixel<OPAQUE>(P, sv, c, x, y);
         }
     }
     if(P.counters)
@@ -167,18 +169,24 @@ namespace {
 // 32-voxel requests (normally the two halves of one chunk's voxel range) from
 // a device work counter.
 
-// Waves per SIMD the lighting kernel is compiled for. At 4 the register
-// allocator keeps 128 VGPRs (a few spills, outside the DDA loops); measured
-// 12% faster than the 154 VGPRs / 3 waves it would take unconstrained.
+// Waves per SIMD the lighting kernel is compiled for, without and with transparent
+// voxels (512x256x512 voxels, every exposed chunk lit; 296x104x232 with glass and
+// mirrors, two samples). Opaque: 3 waves (131 VGPRs) 972 us, 4 (127) 1030, 2 912 but
+// 610 against 530 us in the batch of 24 volumes. General: 5 (96 VGPRs and some 110
+// spilled, outside the walks) 4440 us, 4 (128) 5560, 6 4560, 8 5120.
 #ifndef DN_LIGHT_WAVES
-#define DN_LIGHT_WAVES 4
+#define DN_LIGHT_WAVES 3
+#endif
+#ifndef DN_LIGHT_GENERAL_WAVES
+#define DN_LIGHT_GENERAL_WAVES 5
 #endif
 // Largest chunk-grid occupancy bitmap staged in LDS (bytes): 64 KiB covers
 // 524 288 tiles; bigger maps read it from global memory.
 #define DN_OCC_LDS_MAX 65536u
 
-template <bool LDS_OCC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DN_LIGHT_WAVES, DN_LIGHT_WAVES)))
+template <bool LDS_OCC, bool OPAQUE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OPAQUE ? DN_LIGHT_WAVES : DN_LIGHT_GENERAL_WAVES,
+                                                              OPAQUE ? DN_LIGHT_WAVES : DN_LIGHT_GENERAL_WAVES)))
 void k_lighting(DNlightParams P)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -206,7 +214,7 @@ void k_lighting(DNlightParams P)
         base = __shfl(base, 0, 64);
         if(base >= nreq) break;
         const uint32_t r = base + (lane >> 5);
-        if(r < nreq) light_voxel(P, sv, r, lane & 31u, c, lit, false);
+        if(r < nreq) light_voxel<OPAQUE>(P, sv, r, lane & 31u, c, lit, false);
     }
     if(P.counters)
     {
@@ -233,11 +241,10 @@ void k_lighting(DNlightParams P)
 // with the term (the pass adds them whenever it uses it), so the pass's counts
 // are those of tracing in sequence. Voxels without a diffuse term (specular
 // >= 1) are skipped. A wave takes one request (32 slots) at a time.
-// Waves per SIMD the direct-ray kernel is compiled for: 96 VGPRs, no spills.
-// Measured on the full-frame workload (lighting pass) with the sums spread
-// over 8 lanes per voxel: 4 waves 4.73 ms, 5 waves 4.38, 6 waves (80 VGPRs,
-// a few spills) 4.67, 7 waves 4.67. With one summing lane per voxel 6 waves
-// had been best (4 waves 6.55 ms, 5 waves 5.88, 6 waves 5.49, 7 waves 5.93).
+// Waves per SIMD the direct-ray kernel is compiled for: 5 (81 VGPRs without and 96
+// with transparent voxels, no spills). Every exposed chunk of 512x256x512 voxels, 32
+// directions, opaque: 5 waves 2120 us, 6 2080, 7 2130; the camera's chunks of a 128^3
+// map: 178, 187, 202.
 // The chunk-grid occupancy bitmap is read from L2 here: staging it in LDS
 // (16 KiB per block on that map) would hold the kernel to 4 waves.
 #ifndef DN_DIRECT_WAVES
@@ -252,6 +259,7 @@ void k_lighting(DNlightParams P)
 // The direct rays of one request's 32 slots: lane = voxel * N + direction,
 // 64 / N voxels at a time. `row` is the lane's mask row, `voxRows` the row of
 // its voxel's first direction.
+template <bool OPAQUE>
 __device__ __forceinline__ void direct_request(const DNlightParams& P, const DNsceneView& sv, uint32_t r, RayCtx& c,
                                                uint32_t* row, const uint32_t* voxRows, uint32_t* originRow,
                                                uint32_t N, uint32_t per, uint32_t v, uint32_t k, f3 dir, f3 inv,
@@ -296,7 +304,7 @@ __device__ __forceinline__ void direct_request(const DNlightParams& P, const DNs
             DVoxel hv = {};
             f3 ca;
             float cm;
-            if(!light_trace_uniform(sv, c, dir, inv, pp, hv, ca, cm))
+            if(!light_trace_uniform<OPAQUE>(sv, c, dir, inv, pp, hv, ca, cm))
             {
                 const f3 t = sun * cm + ca;
                 term = make_float4(t.x, t.y, t.z, 1.0f);
@@ -340,6 +348,7 @@ __device__ __forceinline__ void direct_request(const DNlightParams& P, const DNs
     c.sharedMap = 0xFFFFFFFFu;
 }
 
+template <bool OPAQUE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DN_DIRECT_WAVES, DN_DIRECT_WAVES)))
 void k_direct(DNlightParams P)
 {
@@ -366,14 +375,15 @@ void k_direct(DNlightParams P)
         if(lane == 0) r = atomicAdd(P.workCounter + 4, 1u);
         r = __shfl(r, 0, 64);
         if(r >= nreq) break;
-        direct_request(P, sv, r, c, row, voxRows, originRows + (threadIdx.x >> 6) * DN_MASK_ROW, N, per, v, k, dir,
-                       inv, sun);
+        direct_request<OPAQUE>(P, sv, r, c, row, voxRows, originRows + (threadIdx.x >> 6) * DN_MASK_ROW, N, per, v, k,
+                               dir, inv, sun);
     }
 }
 
 // k_direct over the volumes of a batch, with the work units, queues and
 // per-queue counters of k_lighting_batch (its own counters). Volumes whose pass
 // traces its direct rays itself (no directOut) are skipped.
+template <bool OPAQUE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DN_DIRECT_BATCH_WAVES, DN_DIRECT_BATCH_WAVES)))
 void k_direct_batch(DNbatchParams B, const DNlightParams* __restrict__ scenes)
 {
@@ -423,7 +433,7 @@ void k_direct_batch(DNbatchParams B, const DNlightParams* __restrict__ scenes)
             const uint32_t nreq = *P.numRequests;
             const uint32_t r0 = (u - pre[lo]) * B.unit;
             for(uint32_t j = 0; j < B.unit && r0 + j < nreq; j++)
-                direct_request(P, sv, r0 + j, c, row, voxRows, originRows + (threadIdx.x >> 6) * DN_MASK_ROW, N,
+                direct_request<OPAQUE>(P, sv, r0 + j, c, row, voxRows, originRows + (threadIdx.x >> 6) * DN_MASK_ROW, N,
                                per, v, k, dir, inv, sun);
         }
     }
@@ -698,8 +708,9 @@ __device__ __forceinline__ void flush_counters(uint64_t* cnt, RayCtx& c, uint32_
 // Workgroups are dealt to the 8 XCDs round-robin by workgroup id, so with 8
 // queues the home queue of workgroup b is b % 8 and a volume's units stay on
 // one XCD (one L2) while its queue lasts.
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(DN_LIGHT_WAVES, DN_LIGHT_WAVES)))
+template <int BLOCK, bool OPAQUE>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OPAQUE ? DN_LIGHT_WAVES : DN_LIGHT_GENERAL_WAVES,
+                                                              OPAQUE ? DN_LIGHT_WAVES : DN_LIGHT_GENERAL_WAVES)))
 void k_lighting_batch(DNbatchParams B, const DNlightParams* __restrict__ scenes)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -750,7 +761,7 @@ void k_lighting_batch(DNbatchParams B, const DNlightParams* __restrict__ scenes)
             for(uint32_t j = 0; j < B.unit; j += 2u)
             {
                 const uint32_t r = r0 + j + (lane >> 5);
-                if(r < nreq) light_voxel(P, sv, r, lane & 31u, c, lit, dry);
+                if(r < nreq) light_voxel<OPAQUE>(P, sv, r, lane & 31u, c, lit, dry);
             }
         }
     }
@@ -774,7 +785,6 @@ __global__ __launch_bounds__(256) void k_batch_epilogue(const DNlightParams* sce
         epilogue_word(P.scene.flags, (DNchunkRec*)P.scene.chunks, P.litBits, P.visProp, w);
 }
 
-int g_lightingBlocks = 0;
 int g_cus = 0;
 
 int cu_count()
@@ -797,31 +807,35 @@ int cu_count()
 int dn_launch_draw(const DNdrawParams& p, hipStream_t stream)
 {
     // persistent grid of resident blocks, no more than one wave per quad
-    static int perCU = 0;
+    const auto kernel = p.scene.opaque ? k_draw<true> : k_draw<false>;
+    static int perCUs[2] = {0, 0};
+    int& perCU = perCUs[p.scene.opaque ? 1 : 0];
     if(perCU == 0)
     {
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_draw, 256, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kernel, 256, 0);
         if(perCU < 1) perCU = 1;
     }
     const uint32_t quads = ((p.width + 7u) / 8u) * ((p.height + 7u) / 8u);
     uint32_t blocks = (uint32_t)cu_count() * (uint32_t)perCU;
     if((quads + 3u) / 4u < blocks) blocks = (quads + 3u) / 4u;
-    hipLaunchKernelGGL(k_draw, dim3(blocks), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, p);
     return (int)hipGetLastError();
 }
 
 int dn_launch_direct(const DNlightParams& p, uint32_t maxRequests, hipStream_t stream)
 {
     if(p.numDirectRays == 0 || p.numDirectRays > 64u || !p.directOut) return (int)hipErrorInvalidValue;
-    static int perCU = 0;
+    const auto kernel = p.scene.opaque ? k_direct<true> : k_direct<false>;
+    static int perCUs[2] = {0, 0};
+    int& perCU = perCUs[p.scene.opaque ? 1 : 0];
     if(perCU == 0)
     {
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_direct, 256, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kernel, 256, 0);
         if(perCU < 1) perCU = 1;
     }
     uint32_t blocks = (uint32_t)cu_count() * (uint32_t)perCU;
     if(maxRequests / 4 + 1 < blocks) blocks = maxRequests / 4 + 1;
-    hipLaunchKernelGGL(k_direct, dim3(blocks), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, p);
     return (int)hipGetLastError();
 }
 
@@ -829,26 +843,26 @@ int dn_launch_lighting(const DNlightParams& p, uint32_t maxRequests, hipStream_t
 {
     // persistent grid: as many blocks as can be resident with this map's
     // staged bitmap (recomputed when its size changes)
-    static size_t lastOccBytes = ~(size_t)0;
+    static size_t occBytesOf[2] = {~(size_t)0, ~(size_t)0};
+    static int residentOf[2] = {0, 0};
+    const uint32_t v = p.scene.opaque ? 1u : 0u;
     const size_t occBytes = sizeof(uint32_t) * ((p.tiles + 31u) / 32u);
     const bool lds = occBytes <= DN_OCC_LDS_MAX;
-    if(g_lightingBlocks == 0 || occBytes != lastOccBytes)
+    const auto kernel = lds ? (v ? k_lighting<true, true> : k_lighting<true, false>)
+                            : (v ? k_lighting<false, true> : k_lighting<false, false>);
+    if(residentOf[v] == 0 || occBytes != occBytesOf[v])
     {
         int perCU = 0;
-        if(lds) hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_lighting<true>, 256, occBytes);
-        else hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_lighting<false>, 256, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kernel, 256, lds ? occBytes : 0);
         if(perCU < 1) perCU = 1;
-        g_lightingBlocks = cu_count() * perCU;
-        lastOccBytes = occBytes;
+        residentOf[v] = cu_count() * perCU;
+        occBytesOf[v] = occBytes;
     }
     // never more waves than two requests each
     uint32_t needWaves = (maxRequests + 1) / 2;
-    uint32_t blocks = (uint32_t)g_lightingBlocks;
+    uint32_t blocks = (uint32_t)residentOf[v];
     if(needWaves / 4 + 1 < blocks) blocks = needWaves / 4 + 1;
-    if(lds)
-        hipLaunchKernelGGL(k_lighting<true>, dim3(blocks), dim3(256), occBytes, stream, p);
-    else
-        hipLaunchKernelGGL(k_lighting<false>, dim3(blocks), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds ? occBytes : 0, stream, p);
     return (int)hipGetLastError();
 }
 
@@ -874,28 +888,29 @@ int dn_launch_batch(const DNbatchParams& b, uint32_t blockThreads, uint32_t bloc
     hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(1024), 0, stream, b);
     if(direct)
     {
-        static int perCUd = 0;
+        const auto kernel = b.opaque ? k_direct_batch<true> : k_direct_batch<false>;
+        static int perCUds[2] = {0, 0};
+        int& perCUd = perCUds[b.opaque ? 1 : 0];
         if(perCUd == 0)
         {
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCUd, k_direct_batch, 256, 0);
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCUd, kernel, 256, 0);
             if(perCUd < 1) perCUd = 1;
         }
-        hipLaunchKernelGGL(k_direct_batch, dim3((uint32_t)cu_count() * (uint32_t)perCUd), dim3(256), 0, stream, b,
-                           b.scenes);
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)cu_count() * (uint32_t)perCUd), dim3(256), 0, stream, b, b.scenes);
     }
-    static int perCU64 = 0, perCU256 = 0;
-    int& perCU = blockThreads == 64u ? perCU64 : perCU256;
+    const auto kernel = blockThreads == 64u ? (b.opaque ? k_lighting_batch<64, true> : k_lighting_batch<64, false>)
+                                            : (b.opaque ? k_lighting_batch<256, true> : k_lighting_batch<256, false>);
+    static int perCUs[2][2] = {{0, 0}, {0, 0}};
+    int& perCU = perCUs[blockThreads == 64u ? 0 : 1][b.opaque ? 1 : 0];
     if(perCU == 0)
     {
-        if(blockThreads == 64u) hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_lighting_batch<64>, 64, 0);
-        else hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k_lighting_batch<256>, 256, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kernel, (int)blockThreads, 0);
         if(perCU < 1) perCU = 1;
     }
     uint32_t per = (uint32_t)perCU;
     if(blocksPerCU && blocksPerCU < per) per = blocksPerCU;
     const uint32_t blocks = (uint32_t)cu_count() * per;
-    if(blockThreads == 64u) hipLaunchKernelGGL(k_lighting_batch<64>, dim3(blocks), dim3(64), 0, stream, b, b.scenes);
-    else hipLaunchKernelGGL(k_lighting_batch<256>, dim3(blocks), dim3(256), 0, stream, b, b.scenes);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(blockThreads), 0, stream, b, b.scenes);
     if(epilogue && !b.dry)
     {
         uint32_t cx = (maxRequests * 32u + 255u) / 256u;

@@ -898,6 +898,7 @@ __device__ __forceinline__ void site_ctx(const DNlightParams& P, const DNsceneVi
 
 // Lane G draws sample g = G mod n of batch k = G / n, with that batch's seed
 // seed0 + k * seedStride (the batches of several training steps in one launch).
+template <bool OPAQUE>
 __global__ __launch_bounds__(256) void k_rc_samples(DNlightParams P, uint32_t n, uint32_t total, uint32_t seed0,
                                                    uint32_t seedStride, float* samples)
 {
@@ -937,7 +938,7 @@ __global__ __launch_bounds__(256) void k_rc_samples(DNlightParams P, uint32_t n,
     if(mat.specular < 1.0f)
     {
         const SampleRandom rng{base};
-        diffuse_ray(L, v.me.normal + DN_EPS, v.p, v.me, 0, diff, rng);
+        diffuse_ray<OPAQUE>(L, v.me.normal + DN_EPS, v.p, v.me, 0, diff, rng);
         if(!direct_is_exact(P))
         {
             diff = diff + ld3(P.ambient);
@@ -945,13 +946,14 @@ __global__ __launch_bounds__(256) void k_rc_samples(DNlightParams P, uint32_t n,
             DVoxel hv = {};
             f3 ca; float cm;
             f3 pp = v.p;
-            if(!light_trace(s, c, dir, vinv(dir), pp, hv, ca, cm)) diff = diff + (L.sunStrength * cm + ca);
+            if(!light_trace<OPAQUE, !OPAQUE>(s, c, dir, vinv(dir), pp, hv, ca, cm)) diff = diff + (L.sunStrength * cm + ca);
         }
     }
     write_sample(out, v.pos, v.me, diff, 1.0f);
 }
 
 // Query rows for every slot of the request list (valid 0 for empty lanes).
+template <bool OPAQUE>
 __global__ __launch_bounds__(256) void k_rc_gather(DNlightParams P, uint32_t slotsCap, float* samples)
 {
     __shared__ uint32_t maskRows[DN_MASK_LDS_WORDS(256)];
@@ -977,7 +979,7 @@ __global__ __launch_bounds__(256) void k_rc_gather(DNlightParams P, uint32_t slo
         site_ctx(P, s, c, L, maskRows);
         L.direct = (P.directIn && g < P.directSlots) ? P.directIn + g : nullptr;
         exact = ld3(P.ambient);
-        shadow_ray(L, v.p, 0, exact);
+        shadow_ray<OPAQUE>(L, v.p, 0, exact);
     }
     write_sample(out, v.pos, v.me, splat(0.0f), 1.0f, exact);
 }
@@ -986,6 +988,7 @@ __global__ __launch_bounds__(256) void k_rc_gather(DNlightParams P, uint32_t slo
 // thread (per-sample random numbers), `chunks` threads per slot, summed in
 // FP64 into acc[slot] (rgb, sample count). With fixed direct rays each sample
 // is the exact ambient + direct term plus one path-traced indirect term.
+template <bool OPAQUE>
 __global__ __launch_bounds__(256) void k_rc_reference(DNlightParams P, uint32_t slotsCap, uint32_t chunks, uint32_t per,
                                                       uint32_t seed, double* acc)
 {
@@ -1008,14 +1011,14 @@ __global__ __launch_bounds__(256) void k_rc_reference(DNlightParams P, uint32_t 
     if(exactDirect)
     {
         exact = ld3(P.ambient);
-        shadow_ray(L, v.p, 0, exact);
+        shadow_ray<OPAQUE>(L, v.p, 0, exact);
     }
     double sx = 0.0, sy = 0.0, sz = 0.0;
     for(uint32_t k = 0; k < per; k++)
     {
         const SampleRandom rng{pcg(seed ^ pcg(slot * 0x9E3779B9u ^ pcg(chunk * per + k)))};
         f3 smp = splat(0.0f);
-        diffuse_ray(L, v.me.normal + DN_EPS, v.p, v.me, 0, smp, rng);
+        diffuse_ray<OPAQUE>(L, v.me.normal + DN_EPS, v.p, v.me, 0, smp, rng);
         if(exactDirect)
             smp = smp + exact;
         else
@@ -1025,7 +1028,7 @@ __global__ __launch_bounds__(256) void k_rc_reference(DNlightParams P, uint32_t 
             DVoxel hv = {};
             f3 ca; float cm;
             f3 pp = v.p;
-            if(!light_trace(s, c, dir, vinv(dir), pp, hv, ca, cm)) smp = smp + (L.sunStrength * cm + ca);
+            if(!light_trace<OPAQUE, !OPAQUE>(s, c, dir, vinv(dir), pp, hv, ca, cm)) smp = smp + (L.sunStrength * cm + ca);
         }
         sx += (double)smp.x; sy += (double)smp.y; sz += (double)smp.z;
     }
@@ -1144,7 +1147,7 @@ int dn_rc_samples(const DNlightParams& p, uint32_t maxRequests, uint32_t n, uint
     if(n == 0 || batches == 0) return 0;
     if((uint64_t)n * batches > 0xFFFFFFFFull) return (int)hipErrorInvalidValue;
     const uint32_t total = n * batches;
-    hipLaunchKernelGGL(k_rc_samples, dim3(blocks_for(total)), dim3(256), 0, stream, p, n, total, seed, seedStride,
+    hipLaunchKernelGGL(p.scene.opaque ? k_rc_samples<true> : k_rc_samples<false>, dim3(blocks_for(total)), dim3(256), 0, stream, p, n, total, seed, seedStride,
                        samples);
     return (int)hipGetLastError();
 }
@@ -1152,7 +1155,7 @@ int dn_rc_samples(const DNlightParams& p, uint32_t maxRequests, uint32_t n, uint
 int dn_rc_gather(const DNlightParams& p, uint32_t slots, float* samples, hipStream_t stream)
 {
     if(slots == 0) return 0;
-    hipLaunchKernelGGL(k_rc_gather, dim3(blocks_for(slots)), dim3(256), 0, stream, p, slots, samples);
+    hipLaunchKernelGGL(p.scene.opaque ? k_rc_gather<true> : k_rc_gather<false>, dim3(blocks_for(slots)), dim3(256), 0, stream, p, slots, samples);
     return (int)hipGetLastError();
 }
 
@@ -1162,7 +1165,7 @@ int dn_rc_reference(const DNlightParams& p, uint32_t slots, uint32_t samplesPerV
     if(slots == 0 || samplesPerVoxel == 0) return 0;
     const uint32_t chunks = samplesPerVoxel >= 256u ? 16u : 1u;
     const uint32_t per = (samplesPerVoxel + chunks - 1u) / chunks;
-    hipLaunchKernelGGL(k_rc_reference, dim3(blocks_for((size_t)slots * chunks)), dim3(256), 0, stream, p, slots, chunks,
+    hipLaunchKernelGGL(p.scene.opaque ? k_rc_reference<true> : k_rc_reference<false>, dim3(blocks_for((size_t)slots * chunks)), dim3(256), 0, stream, p, slots, chunks,
                        per, seed, acc);
     return (int)hipGetLastError();
 }
