@@ -88,3 +88,32 @@ def test_batch_with_one_transparent_volume(gpu):
     batch.close()
     for v in va + vb:
         v.close()
+
+
+@pytest.mark.parametrize("visible", [1, 2, 7, 100000])
+@pytest.mark.parametrize("n_direct", [1, 5, 16, 33, 64])
+def test_direct_rays_in_parts_of_requests(gpu, n_direct, visible):
+    """Few requests: a single volume's direct rays go to the waves in parts of a
+    request, a batch's in whole requests."""
+    sc = scenes.batch_scene(4, max_grid=8)
+    vols = []
+    for _ in range(2):
+        v = Volume(sc.map_size, min_chunks=64)
+        sc.apply(v)
+        v.v.numDirectRays = n_direct
+        v.request_all()
+        v.sync()
+        v.mark_visible(visible)
+        v.sync()
+        vols.append(v)
+    batch = Batch(vols[1:])
+    for f in range(2):
+        vols[0].update_lighting(1, 1000, 20.0 + f)
+        batch.update_lighting(1, 1000, 20.0 + f)
+        assert_same(vols[:1], vols[1:], f"frame {f}")
+        for v in vols:
+            v.mark_visible(visible)
+            v.sync()
+    batch.close()
+    for v in vols:
+        v.close()
