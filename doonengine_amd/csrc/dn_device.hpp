@@ -710,10 +710,25 @@ __device__ __forceinline__ f3 sky_color(const DNsceneView& s, f3 dir)
     return vmix(ld3(s.skyBot), ld3(s.skyTop), dir.y * 0.5f + 1.0f);
 }
 
-// wave-wide sum and one atomic per wave into a u64 counter
-__device__ __forceinline__ void wave_add_u64(uint64_t* dst, uint32_t v)
+// Adds a wave's counts to the counters of its kind: lane k adds the wave's sum of
+// count k, all with one instruction into one cache line. Atomics on a line are
+// served one after the other, some 15 ns each, also for counts that nothing waits
+// for, so the counters are kept in copies, which the blocks use in turn.
+__device__ __forceinline__ void wave_add_counts(uint64_t* counters, RayCtx& c, uint32_t lit, uint32_t pixels)
 {
-    uint64_t x = v;
-    for(int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-    if((threadIdx.x & 63u) == 0 && x) atomicAdd((unsigned long long*)dst, (unsigned long long)x);
+    if(!counters) return;
+    const uint32_t counts[6] = {c.cRays, c.cMap, c.cVox, c.cHits, lit, pixels};
+    static_assert(CNT_RAYS == 0 && CNT_MAPSTEPS == 1 && CNT_VOXSTEPS == 2 && CNT_HITS == 3 && CNT_LIT == 4 &&
+                      CNT_PIXELS == 5, "slots in the order of the counts");
+    const uint32_t lane = threadIdx.x & 63u;
+    uint64_t mine = 0;
+    for(uint32_t k = 0; k < 6u; k++)
+    {
+        uint64_t x = counts[k];
+        for(int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+        if(lane == k) mine = x;
+    }
+    if(mine)
+        atomicAdd((unsigned long long*)(counters + (size_t)(blockIdx.x % CNT_COPIES) * CNT_STRIDE + lane),
+                  (unsigned long long)mine);
 }

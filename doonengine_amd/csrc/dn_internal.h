@@ -59,6 +59,19 @@ struct DNsceneView {
     const int32_t* colTop;
 };
 
+// Counter slots (u64 each) per kind.
+// They are kept in CNT_COPIES copies, CNT_STRIDE slots (4 kinds) apart, whose sum
+// is the count.
+enum { CNT_RAYS = 0, CNT_MAPSTEPS, CNT_VOXSTEPS, CNT_HITS, CNT_LIT, CNT_PIXELS, CNT_SLOTS = 8, CNT_COPIES = 32,
+       CNT_STRIDE = 4 * CNT_SLOTS };
+
+// A volume's work counters (u32): the tickets of the lighting pass, of its direct
+// rays and of the draw, each in DN_TICKET_LINES cache lines that the blocks use in
+// turn, then the draw's finished blocks and the collected requests.
+enum { DN_TICKET_LINES = 8, DN_LINE_WORDS = 32, WORK_LIGHT = 0, WORK_DIRECT = DN_TICKET_LINES * DN_LINE_WORDS,
+       WORK_DRAW = 2 * WORK_DIRECT, WORK_DONE = 3 * WORK_DIRECT, WORK_COLLECTED = WORK_DONE + DN_LINE_WORDS,
+       WORK_WORDS = WORK_COLLECTED + DN_LINE_WORDS };
+
 // Limits of the per-frame tables passed by value to the lighting kernel.
 enum { DN_MAX_POINTS = 64, DN_MAX_SAMPLES = 4, DN_MAX_BOUNCES = 8 };
 
@@ -86,7 +99,7 @@ struct DNlightParams {
     DNsceneView scene;
     const uint32_t* requests;
     const uint32_t* numRequests;   // device count
-    uint32_t* workCounter;         // device, reset by the epilogue
+    uint32_t* workCounter;         // device (WORK_*), its tickets reset by the epilogue
     uint32_t* litBits;             // bit per tile, set for lit chunks
     uint32_t* visProp;             // bit per tile, set by specular rays
     uint4* voxelsOut;              // pool receiving lit words (== voxels when written in place)
@@ -133,8 +146,8 @@ struct DNbatchParams {
     uint32_t opaque;               // every volume is (DNsceneView::opaque)
     uint32_t dry;                  // 1: compute only, no stores (autotuning)
     uint32_t* dryLastUsed;         // dry: where rays' lastUsed stores go instead (>= the largest volume's tiles)
-    uint32_t* queueCounters;       // [queues] next unit of each queue
-    uint32_t* directCounters;      // [queues] next unit of each queue for the direct-ray pass
+    uint32_t* queueCounters;       // [queues] next unit of each queue, DN_LINE_WORDS apart
+    uint32_t* directCounters;      // the same for the direct-ray pass
     const uint32_t* queueScenes;   // [queues][numScenes] volume ids of each queue, in order
     const uint32_t* queueLen;      // [queues] volumes in each queue
     uint32_t* queuePrefix;         // [queues][numScenes + 1] exclusive unit prefix, written on device
@@ -149,7 +162,7 @@ struct DNdrawParams {
     float4* out;
     void* hitOut;                  // optional DNXpixelHit*
     uint64_t* counters;
-    uint32_t* quadCounter;         // device [2]: next 8x8 quad, finished waves; zero between launches
+    uint32_t* workCounter;         // device (WORK_*); its draw tickets and finished blocks are zero between launches
 };
 
 struct DNrayParams {
@@ -183,9 +196,6 @@ struct DNvisibleParams {
     uint32_t* requests;
     uint32_t* numRequests;
 };
-
-// Counter slots (u64 each) per kind.
-enum { CNT_RAYS = 0, CNT_MAPSTEPS, CNT_VOXSTEPS, CNT_HITS, CNT_LIT, CNT_PIXELS, CNT_SLOTS = 8 };
 
 // Device sphere edits (edits.hip). A batch of spheres is split into (tile,
 // sphere) pairs, numbered in the reference's order (sphere by sphere, tiles of

@@ -141,12 +141,11 @@ struct DNgpuVolume {
     int32_t* dColTop = nullptr;        // DNsceneView::colTop, 4 x mapZ x mapX
     size_t colTopCap = 0;              // in entries
     bool colTopValid = false;          // dColTop holds the tables of the present state
-    uint32_t* dWorkCounter = nullptr;  // [0] lighting requests taken, [1] collected requests, [2..3] draw quads,
-                                       // [4] direct-ray requests taken
+    uint32_t* dWorkCounter = nullptr;  // WORK_*
     DNdirectTerm* dDirect = nullptr;   // direct-ray terms per request slot (k_direct)
     size_t directCap = 0;              // in slots
     uint32_t* dReqList = nullptr;      // tiles requested by rays (collect)
-    uint64_t* dCounters = nullptr;     // 3 kinds x CNT_SLOTS
+    uint64_t* dCounters = nullptr;     // CNT_COPIES x CNT_STRIDE, 3 kinds x CNT_SLOTS of each in use
     float* dPoints = nullptr;          // 2 x DN_MAX_POINTS x 3
     uint32_t specN = 0, directN = 0;
     std::vector<float> specPts, directPts;
@@ -779,7 +778,7 @@ bool collect_ray_requests(DNvolume* vol)
     DNgpuVolume* g = vol->gpu;
     // after every sync each tile is 0, 1 or 2, so numUnloaded counts state-1 tiles
     if(g->numUnloaded == 0) return true;
-    uint32_t* dCount = g->dWorkCounter + 1;
+    uint32_t* dCount = g->dWorkCounter + WORK_COLLECTED;
     if(!HIP_OK(hipMemsetAsync(dCount, 0, sizeof(uint32_t), g->stream), "ray request count")) return false;
     int e = dn_launch_collect_requested(g->dFlags, g->tiles, g->dReqList, dCount, g->stream);
     if(e)
@@ -895,8 +894,8 @@ extern "C" DNvolume* DN_create_volume(DNuvec3 mapSize, unsigned int minChunks)
     const uint32_t tiles = mapSize.x * mapSize.y * mapSize.z;
     if(!HIP_OK(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking), "stream") ||
        !alloc_tile_buffers(g, tiles) || !dalloc(&g->dMats, DN_MAX_MATERIALS, "material buffer") ||
-       !dalloc(&g->dNumRequests, 1, "request count") || !dalloc(&g->dWorkCounter, 6, "work counter") ||
-       !dalloc(&g->dCounters, 3 * CNT_SLOTS, "counters") || !dalloc(&g->dPoints, 2 * DN_MAX_POINTS * 3, "ray table") ||
+       !dalloc(&g->dNumRequests, 1, "request count") || !dalloc(&g->dWorkCounter, WORK_WORDS, "work counter") ||
+       !dalloc(&g->dCounters, CNT_COPIES * CNT_STRIDE, "counters") || !dalloc(&g->dPoints, 2 * DN_MAX_POINTS * 3, "ray table") ||
        !HIP_OK(hipHostMalloc((void**)&g->hSmall, 64, hipHostMallocDefault), "pinned readback") ||
        !HIP_OK(hipEventCreate(&g->stageDone[0]), "event") || !HIP_OK(hipEventCreate(&g->stageDone[1]), "event"))
     {
@@ -904,8 +903,8 @@ extern "C" DNvolume* DN_create_volume(DNuvec3 mapSize, unsigned int minChunks)
         return nullptr;
     }
     if(!HIP_OK(hipMemsetAsync(g->dNumRequests, 0, sizeof(uint32_t), g->stream), "request count") ||
-       !HIP_OK(hipMemsetAsync(g->dWorkCounter, 0, 6 * sizeof(uint32_t), g->stream), "work counter") ||
-       !HIP_OK(hipMemsetAsync(g->dCounters, 0, 3 * CNT_SLOTS * sizeof(uint64_t), g->stream), "counters") ||
+       !HIP_OK(hipMemsetAsync(g->dWorkCounter, 0, WORK_WORDS * sizeof(uint32_t), g->stream), "work counter") ||
+       !HIP_OK(hipMemsetAsync(g->dCounters, 0, CNT_COPIES * CNT_STRIDE * sizeof(uint64_t), g->stream), "counters") ||
        !HIP_OK(hipMemsetAsync(g->dMats, 0, sizeof(DNmat) * DN_MAX_MATERIALS, g->stream), "material buffer"))
     {
         DN_delete_volume(vol);
@@ -1467,7 +1466,7 @@ extern "C" void DN_draw(DNvolume* vol, DNtexture out, DNmat4 view, DNmat4 projec
     if(g->drawHitOut && !p.hitOut)
         dn_msg(DN_MESSAGE_GPU_MEMORY, DN_MESSAGE_ERROR, "draw hit output smaller than the image; not written");
     p.counters = g->dCounters + 0 * CNT_SLOTS;
-    p.quadCounter = g->dWorkCounter + 2;
+    p.workCounter = g->dWorkCounter;
     Timer tm = timer_begin(g, TK_DRAW);
     int e = dn_launch_draw(p, g->stream);
     timer_end(g, tm);
@@ -1584,9 +1583,10 @@ bool trace_direct_terms(DNvolume* vol, DNlightParams& p, uint32_t maxRequests)
     p.directSlots = (uint32_t)std::min<size_t>(g->directCap, 0xFFFFFFFFu);
     const int e = dn_launch_direct(p, maxRequests, g->stream);
     p.directOut = nullptr;
-    // k_direct's request counter, which the lighting pass's epilogue clears
+    // k_direct's tickets, which the lighting pass's epilogue clears
     // otherwise (this runs outside a lighting pass and outside graph capture)
-    const bool ok = e == 0 && HIP_OK(hipMemsetAsync(g->dWorkCounter + 4, 0, sizeof(uint32_t), g->stream), "counter");
+    const bool ok = e == 0 && HIP_OK(hipMemsetAsync(g->dWorkCounter + WORK_DIRECT, 0,
+                                                    DN_TICKET_LINES * DN_LINE_WORDS * sizeof(uint32_t), g->stream), "counter");
     if(ok) p.directIn = g->dDirect;
     else p.directSlots = 0;
     return ok;
@@ -2750,13 +2750,15 @@ extern "C" void DNX_get_counters(DNvolume* vol, int kind, DNXcounters* out, bool
 {
     DNgpuVolume* g = vol->gpu;
     if(kind < 0 || kind > 2) { memset(out, 0, sizeof(*out)); return; }
-    uint64_t c[CNT_SLOTS];
+    uint64_t all[CNT_COPIES * CNT_STRIDE], c[CNT_SLOTS] = {};
     if(!HIP_OK(hipStreamSynchronize(g->stream), "counters") ||
-       !HIP_OK(hipMemcpy(c, g->dCounters + kind * CNT_SLOTS, sizeof(c), hipMemcpyDeviceToHost), "counters"))
+       !HIP_OK(hipMemcpy(all, g->dCounters, sizeof(all), hipMemcpyDeviceToHost), "counters"))
     {
         memset(out, 0, sizeof(*out));
         return;
     }
+    for(int copy = 0; copy < CNT_COPIES; copy++)
+        for(int k = 0; k < CNT_SLOTS; k++) c[k] += all[copy * CNT_STRIDE + kind * CNT_SLOTS + k];
     out->rays = c[CNT_RAYS];
     out->mapSteps = c[CNT_MAPSTEPS];
     out->voxelSteps = c[CNT_VOXSTEPS];
@@ -2765,7 +2767,8 @@ extern "C" void DNX_get_counters(DNvolume* vol, int kind, DNXcounters* out, bool
     out->pixels = c[CNT_PIXELS];
     if(reset)
     {
-        hipMemset(g->dCounters + kind * CNT_SLOTS, 0, sizeof(c));
+        hipMemset2D(g->dCounters + kind * CNT_SLOTS, CNT_STRIDE * sizeof(uint64_t), 0, CNT_SLOTS * sizeof(uint64_t),
+                    CNT_COPIES);
         hipDeviceSynchronize();
     }
 }
@@ -2928,7 +2931,7 @@ DNbatchParams batch_params(DNXbatch* b, bool dry)
     bp.opaque = b->allOpaque ? 1u : 0u;
     bp.dry = dry ? 1u : 0u;
     bp.queueCounters = b->dQueueCounters;
-    bp.directCounters = b->dQueueCounters + DN_BATCH_MAX_QUEUES;
+    bp.directCounters = b->dQueueCounters + DN_BATCH_MAX_QUEUES * DN_LINE_WORDS;
     bp.queueScenes = b->dQueueScenes;
     bp.queueLen = b->dQueueLen;
     bp.queuePrefix = b->dQueuePrefix;
@@ -3008,7 +3011,7 @@ extern "C" DNXbatch* DNX_batch_create(DNvolume* const* volumes, uint32_t count)
                     "batch parameters") &&
              HIP_OK(hipEventCreateWithFlags(&b->slotDone[s], hipEventDisableTiming), "batch event");
     ok = ok && dalloc(&b->dParams, count, "batch parameters") &&
-         dalloc(&b->dQueueCounters, 2 * DN_BATCH_MAX_QUEUES, "batch queues") &&
+         dalloc(&b->dQueueCounters, 2 * DN_BATCH_MAX_QUEUES * DN_LINE_WORDS, "batch queues") &&
          dalloc(&b->dQueueScenes, (size_t)DN_BATCH_MAX_QUEUES * count, "batch queues") &&
          dalloc(&b->dQueueLen, DN_BATCH_MAX_QUEUES, "batch queues") &&
          dalloc(&b->dQueuePrefix, (size_t)DN_BATCH_MAX_QUEUES * (count + 1u), "batch queues");

@@ -92,8 +92,46 @@ __device__ __forceinline__ void draw_pixel(const DNdrawParams& P, const DNsceneV
     if(P.hitOut) reinterpret_cast<PixelHit*>(P.hitOut)[o] = info;
 }
 
-// Persistent draw: each wave takes 8x8 pixel quads (numbered row by row) from
-// a device counter, lane l drawing pixel (l & 7, l >> 3) of the quad. Chunk
+// The units of a persistent launch, dealt to its waves. Wave w's first unit is w,
+// counted over the blocks before the waves of a block, so that a launch with fewer
+// units than waves spreads over all CUs (taken from a counter, they went to whichever
+// blocks had started). The others are taken by tickets of a device counter. Atomics on
+// one cache line are served one after the other, some 15 ns each over the 8 XCDs, so
+// there are DN_TICKET_LINES of them, which the blocks use in turn, line g for the units
+// g, g + 8, ...; and where units are short and many (`fours`) the first 7/8 go four
+// at a time.
+struct WaveUnits {
+    uint32_t* counter;
+    uint32_t waves, units, quads, next, left, lines;
+    __device__ __forceinline__ WaveUnits(uint32_t* counter_, uint32_t units_, bool fours)
+        : units(units_)
+    {
+        waves = gridDim.x * (blockDim.x >> 6);
+        const uint32_t rest = units > waves ? units - waves : 0u;
+        quads = fours && rest >= 16u * waves ? rest / 32u * 7u : 0u;
+        next = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+        left = 1u;
+        lines = min(gridDim.x, (uint32_t)DN_TICKET_LINES);
+        counter = counter_ + blockIdx.x % lines * DN_LINE_WORDS;
+    }
+    // the next unit of the calling wave; false once there is none
+    __device__ __forceinline__ bool take(uint32_t& u)
+    {
+        if(left == 0u)
+        {
+            uint32_t t = 0;
+            if((threadIdx.x & 63u) == 0u) t = atomicAdd(counter, 1u);
+            t = __builtin_amdgcn_readfirstlane(t) * lines + blockIdx.x % lines;
+            left = t < quads ? 4u : 1u;
+            next = waves + (t < quads ? 4u * t : 3u * quads + t);
+        }
+        u = next++;
+        left--;
+        return u < units;
+    }
+};
+
+// Persistent draw: each wave takes 8x8 pixel quads (numbered row by row), lane l drawing pixel (l & 7, l >> 3) of the quad. Chunk
 // masks go to per-lane LDS rows on chunk entry; the chunk-grid occupancy bits
 // are read through L2 (staging the bitmap in LDS per block measured 0.75 vs
 // 0.71 ms at 1920x1080: neighbouring primary rays read the same words). The
@@ -114,20 +152,19 @@ void k_draw(DNdrawParams P)
     const uint32_t qx = (P.width + 7u) / 8u, nq = qx * ((P.height + 7u) / 8u);
     uint32_t drawn = 0;
     // The first 3/4 of the quads are dealt out statically (wave w takes quads
-    // w, w + W, w + 2W, ...) and the rest from the device counter, in order,
-    // to even out the waves' ends. Every quad from the counter costs one
-    // atomic on that single word, which all 8 XCDs share; at one atomic per
-    // quad those serialise to a floor of about 0.5 ms per 1920x1080 frame
-    // (0.70 ms measured against 0.52 ms with the static share).
+    // w, w + W, w + 2W, ...) and the rest by tickets, to even out the waves' ends
+    // (tickets in lines as in WaveUnits).
     const uint32_t waves = gridDim.x * 4u, wave = blockIdx.x * 4u + (threadIdx.x >> 6);
     const uint32_t perWave = (nq / 4u * 3u) / waves, head = perWave * waves;
+    const uint32_t lines = min(gridDim.x, (uint32_t)DN_TICKET_LINES), line = blockIdx.x % lines;
+    uint32_t* tickets = P.workCounter + WORK_DRAW;
     for(uint32_t k = 0;; k++)
     {
         uint32_t q = wave + k * waves;
         if(k >= perWave)
         {
-            if(lane == 0) q = atomicAdd(P.quadCounter, 1u);
-            q = __shfl(q, 0, 64) + head;
+            if(lane == 0) q = atomicAdd(tickets + line * DN_LINE_WORDS, 1u);
+            q = __builtin_amdgcn_readfirstlane(q) * lines + line + head;
         }
         if(q >= nq) break;
         const uint32_t x = (q % qx) * 8u + (lane & 7u), y = (q / qx) * 8u + (lane >> 3);
@@ -137,23 +174,17 @@ void k_draw(DNdrawParams P)
             draw_pixel<OPAQUE>(P, sv, c, x, y);
         }
     }
-    if(P.counters)
+    wave_add_counts(P.counters, c, 0u, drawn);
+    // the last block to finish, all its waves having taken their last quads, clears
+    // the tickets for the next launch
+    __syncthreads();
+    if(threadIdx.x == 0)
     {
-        wave_add_u64(P.counters + CNT_RAYS, c.cRays);
-        wave_add_u64(P.counters + CNT_MAPSTEPS, c.cMap);
-        wave_add_u64(P.counters + CNT_VOXSTEPS, c.cVox);
-        wave_add_u64(P.counters + CNT_HITS, c.cHits);
-        wave_add_u64(P.counters + CNT_PIXELS, drawn);
-    }
-    if(lane == 0)
-    {
-        // every wave has taken its last quad before it counts itself out
         __threadfence();
-        const uint32_t done = atomicAdd(P.quadCounter + 1, 1u);
-        if(done == gridDim.x * 4u - 1u)
+        if(atomicAdd(P.workCounter + WORK_DONE, 1u) == gridDim.x - 1u)
         {
-            atomicExch(P.quadCounter, 0u);
-            atomicExch(P.quadCounter + 1, 0u);
+            for(uint32_t g = 0; g < DN_TICKET_LINES; g++) atomicExch(tickets + g * DN_LINE_WORDS, 0u);
+            atomicExch(P.workCounter + WORK_DONE, 0u);
         }
     }
 }
@@ -168,41 +199,6 @@ namespace {
 // lighting pass: one lane per stored voxel; a wave takes two consecutive
 // 32-voxel requests (normally the two halves of one chunk's voxel range) from
 // a device work counter.
-
-// The units of a persistent launch, dealt to its waves. Wave w's first unit is w,
-// counted over the blocks before the waves of a block, so that a launch with fewer
-// units than waves spreads over all CUs (taken from a counter, they went to whichever
-// blocks had started). The others are taken from a device counter. Atomics on one word
-// that the 8 XCDs share are served one after the other, some 15 ns each: where units
-// are short and many (`fours`), the first 7/8 go four at a time.
-struct WaveUnits {
-    uint32_t* counter;
-    uint32_t waves, units, quads, next, left;
-    __device__ __forceinline__ WaveUnits(uint32_t* counter_, uint32_t units_, bool fours)
-        : counter(counter_), units(units_)
-    {
-        waves = gridDim.x * (blockDim.x >> 6);
-        const uint32_t rest = units > waves ? units - waves : 0u;
-        quads = fours && rest >= 16u * waves ? rest / 32u * 7u : 0u;
-        next = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-        left = 1u;
-    }
-    // the next unit of the calling wave; false once there is none
-    __device__ __forceinline__ bool take(uint32_t& u)
-    {
-        if(left == 0u)
-        {
-            uint32_t t = 0;
-            if((threadIdx.x & 63u) == 0u) t = atomicAdd(counter, 1u);
-            t = __builtin_amdgcn_readfirstlane(t);
-            left = t < quads ? 4u : 1u;
-            next = waves + (t < quads ? 4u * t : 3u * quads + t);
-        }
-        u = next++;
-        left--;
-        return u < units;
-    }
-};
 
 // Waves per SIMD the lighting kernel is compiled for, without and with transparent
 // voxels (512x256x512 voxels, every exposed chunk lit; 296x104x232 with glass and
@@ -246,20 +242,13 @@ void k_lighting(DNlightParams P)
     // where every exposed chunk of 512x256x512 voxels is lit (one atomic in 7 is left);
     // not with specular materials, whose voxels trace up to 15 times the rays of others
     // (296x104x232 with mirrors: 7100 against 4840 us).
-    WaveUnits work(P.workCounter, (nreq + 1u) / 2u, P.copyBack == 0u);
+    WaveUnits work(P.workCounter + WORK_LIGHT, (nreq + 1u) / 2u, P.copyBack == 0u);
     for(uint32_t u; work.take(u);)
     {
         const uint32_t r = 2u * u + (lane >> 5);
         if(r < nreq) light_voxel<OPAQUE>(P, sv, r, lane & 31u, c, lit, false);
     }
-    if(P.counters)
-    {
-        wave_add_u64(P.counters + CNT_RAYS, c.cRays);
-        wave_add_u64(P.counters + CNT_MAPSTEPS, c.cMap);
-        wave_add_u64(P.counters + CNT_VOXSTEPS, c.cVox);
-        wave_add_u64(P.counters + CNT_HITS, c.cHits);
-        wave_add_u64(P.counters + CNT_LIT, lit);
-    }
+    wave_add_counts(P.counters, c, lit, 0u);
 }
 
 // Direct rays of the pass's voxels, traced ahead of k_lighting. The N direct
@@ -413,7 +402,7 @@ void k_direct(DNlightParams P)
     uint32_t parts = 1u;
     while(parts < groups && nreq * parts * 2u <= waves) parts *= 2u;
     const uint32_t span = (groups + parts - 1u) / parts * per;
-    WaveUnits work(P.workCounter + 4, nreq * parts, false);
+    WaveUnits work(P.workCounter + WORK_DIRECT, nreq * parts, false);
     for(uint32_t u; work.take(u);)
     {
         const uint32_t r = u / parts, first = (u - r * parts) * span;
@@ -448,7 +437,7 @@ void k_direct_batch(DNbatchParams B, const DNlightParams* __restrict__ scenes)
         for(;;)
         {
             uint32_t u = 0;
-            if(lane == 0) u = atomicAdd(&B.directCounters[q], 1u);
+            if(lane == 0) u = atomicAdd(B.directCounters + q * DN_LINE_WORDS, 1u);
             u = __builtin_amdgcn_readfirstlane(__shfl(u, 0, 64));
             if(u >= total) break;
             uint32_t lo = 0, hi = len - 1u;           // last volume with pre[i] <= u
@@ -505,12 +494,16 @@ __device__ __forceinline__ void epilogue_word(uint32_t* flags, DNchunkRec* chunk
     visProp[w] = 0u;
 }
 
-// The epilogue of one pass; also resets the pass's work counter.
+// The epilogue of one pass; also resets the pass's tickets.
 __global__ __launch_bounds__(256) void k_light_epilogue(uint32_t* flags, DNchunkRec* chunks, uint32_t* litBits,
                                                         uint32_t* visProp, uint32_t words, uint32_t* workCounter)
 {
     const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-    if(w == 0) { workCounter[0] = 0u; workCounter[4] = 0u; }
+    if(w < DN_TICKET_LINES)
+    {
+        workCounter[WORK_LIGHT + w * DN_LINE_WORDS] = 0u;
+        workCounter[WORK_DIRECT + w * DN_LINE_WORDS] = 0u;
+    }
     if(w < words) epilogue_word(flags, chunks, litBits, visProp, w);
 }
 
@@ -663,13 +656,7 @@ __global__ __launch_bounds__(256) void k_rays(DNrayParams P)
         o.normal[0] = nrm.x; o.normal[1] = nrm.y; o.normal[2] = nrm.z;
         reinterpret_cast<RayHit*>(P.out)[i] = o;
     }
-    if(P.counters)
-    {
-        wave_add_u64(P.counters + CNT_RAYS, c.cRays);
-        wave_add_u64(P.counters + CNT_MAPSTEPS, c.cMap);
-        wave_add_u64(P.counters + CNT_VOXSTEPS, c.cVox);
-        wave_add_u64(P.counters + CNT_HITS, c.cHits);
-    }
+    wave_add_counts(P.counters, c, 0u, 0u);
 }
 
 __global__ __launch_bounds__(256) void k_collect_requested(const uint32_t* flags, uint32_t tiles, uint32_t* list,
@@ -704,7 +691,11 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(DNbatchParams B)
     __shared__ uint32_t waveSums[16];
     __shared__ uint32_t carry;
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-    if(t < B.queues) { B.queueCounters[t] = 0u; B.directCounters[t] = 0u; }
+    if(t < B.queues)
+    {
+        B.queueCounters[t * DN_LINE_WORDS] = 0u;
+        B.directCounters[t * DN_LINE_WORDS] = 0u;
+    }
     for(uint32_t q = 0; q < B.queues; q++)
     {
         const uint32_t len = B.queueLen[q];
@@ -734,14 +725,7 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(DNbatchParams B)
 
 __device__ __forceinline__ void flush_counters(uint64_t* cnt, RayCtx& c, uint32_t& lit)
 {
-    if(cnt)
-    {
-        wave_add_u64(cnt + CNT_RAYS, c.cRays);
-        wave_add_u64(cnt + CNT_MAPSTEPS, c.cMap);
-        wave_add_u64(cnt + CNT_VOXSTEPS, c.cVox);
-        wave_add_u64(cnt + CNT_HITS, c.cHits);
-        wave_add_u64(cnt + CNT_LIT, lit);
-    }
+    wave_add_counts(cnt, c, lit, 0u);
     c.cRays = c.cMap = c.cVox = c.cHits = 0;
     lit = 0;
 }
@@ -775,7 +759,7 @@ void k_lighting_batch(DNbatchParams B, const DNlightParams* __restrict__ scenes)
         for(;;)
         {
             uint32_t u = 0;
-            if(lane == 0) u = atomicAdd(&B.queueCounters[q], 1u);
+            if(lane == 0) u = atomicAdd(B.queueCounters + q * DN_LINE_WORDS, 1u);
             u = __builtin_amdgcn_readfirstlane(__shfl(u, 0, 64));
             if(u >= total) break;
             uint32_t lo = 0, hi = len - 1u;           // last volume with pre[i] <= u
