@@ -441,12 +441,17 @@ __device__ __forceinline__ bool step_chunk_opaque(const DNsceneView& s, RayCtx& 
 
 // step_map, voxelShared.comp:421-475. LIGHT: a lighting ray, which does not refract
 // and ends once it can meet nothing more (below). OPAQUE: every stored voxel is
-// opaque. VOXEL: false leaves out what the ray hit (`vox` and c.hitIndex).
-template <bool LIGHT, bool OPAQUE, bool FINITE = false, bool VOXEL = true>
+// opaque. VOXEL: false leaves out what the ray hit (`vox` and c.hitIndex). TOGETHER:
+// the trips over tiles that are not loaded are a loop of their own, which a wave
+// leaves once all its lanes are at a loaded tile or out of the map. That pays for rays
+// that have nothing in common; neighbouring rays meet the same tiles at the same
+// trips, and a frame's lighting took 22% longer with it.
+template <bool LIGHT, bool OPAQUE, bool FINITE = false, bool VOXEL = true, bool TOGETHER = false>
 __device__ bool step_map(const DNsceneView& s, RayCtx& c, f3& dir, f3 inv, f3& p, bool ignoreFirst, f3& hitNormal,
                          DVoxel& vox, f3& colorAdd, float& colorMult)
 {
     static_assert(OPAQUE || VOXEL, "transparent voxels are looked up on the way");
+    static_assert(!(LIGHT && TOGETHER), "no stop rules between loaded tiles");
     constexpr bool REFRACT = !LIGHT && !OPAQUE;
     bool requested = false;
     colorAdd = splat(0.0f);
@@ -467,7 +472,32 @@ __device__ bool step_map(const DNsceneView& s, RayCtx& c, f3& dir, f3 inv, f3& p
         c.sMap++;
         const int32_t colTop = colRule ? s.colTop[colBase + (uint32_t)d.px + s.mapX * (uint32_t)d.pz] : INT32_MAX;
         idx = (uint32_t)d.px + s.mapX * ((uint32_t)d.py + s.mapY * (uint32_t)d.pz);
-        if(occ_bit(s.occLoaded, idx))
+        bool loaded = occ_bit(s.occLoaded, idx);
+        if constexpr(TOGETHER)
+        {
+            bool on = true;
+            while(!loaded && on)
+            {
+                if(s.hasUnloaded && !requested && occ_bit(s.occPresent, idx))
+                {
+                    s.flags[idx] = 3u;
+                    requested = true;
+                }
+                lsd.set(d.side);
+                if(FINITE) iterate_dda_finite(d, hitNormal);
+                else iterate_dda(d, hitNormal);
+                ignoreFirst = false;
+                on = in_map_cell(d, (uint32_t)X, (uint32_t)Y, (uint32_t)Z);
+                if(on)
+                {
+                    c.sMap++;
+                    idx = (uint32_t)d.px + s.mapX * ((uint32_t)d.py + s.mapY * (uint32_t)d.pz);
+                    loaded = occ_bit(s.occLoaded, idx);
+                }
+            }
+            if(!loaded) break;
+        }
+        if(loaded)
         {
             s.lastUsed[idx] = 0u;          // a plain store: no read on the ray's path
             f3 upd = p + dir * (lsd.minc() - DN_EPS);
@@ -533,8 +563,8 @@ __device__ bool step_map(const DNsceneView& s, RayCtx& c, f3& dir, f3 inv, f3& p
 // trip ends with the same `lsd = side; iterate` for every lane whatever its
 // level, and only the occupancy test differs: lanes of a wave stay converged
 // instead of waiting on each other's inner chunk loops. The sequence of
-// floating-point operations per ray is exactly that of step_map<false>
-// (voxelShared.comp:328-475): map state is saved on chunk entry and resumed,
+// floating-point operations per ray is exactly that of step_map without
+// refraction (voxelShared.comp:328-475): map state is saved on chunk entry and resumed,
 // then stepped, when the chunk walk leaves the chunk.
 // With NORMAL, hitNormal receives the face normal of the last step taken (the
 // value iterate_dda leaves in it), computed once from the last step mask.

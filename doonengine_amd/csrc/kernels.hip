@@ -67,7 +67,9 @@ __device__ __forceinline__ void draw_pixel(const DNdrawParams& P, const DNsceneV
         f3 nrm = vnorm(tr);
         DVoxel vox = {};
         f3 ca; float cm;
-        bool hit = step_map<false, OPAQUE>(s, c, dir, inv, p, false, nrm, vox, ca, cm);
+        bool hit;
+        if(OPAQUE && all_finite(inv)) hit = step_map<false, OPAQUE, OPAQUE>(s, c, dir, inv, p, false, nrm, vox, ca, cm);
+        else hit = step_map<false, OPAQUE>(s, c, dir, inv, p, false, nrm, vox, ca, cm);
         info.mapSteps = c.sMap; info.voxelSteps = c.sVox;
         if(hit)
         {
@@ -131,16 +133,17 @@ struct WaveUnits {
     }
 };
 
-// Persistent draw: each wave takes 8x8 pixel quads (numbered row by row), lane l drawing pixel (l & 7, l >> 3) of the quad. Chunk
-// masks go to per-lane LDS rows on chunk entry; the chunk-grid occupancy bits
-// are read through L2 (staging the bitmap in LDS per block measured 0.75 vs
-// 0.71 ms at 1920x1080: neighbouring primary rays read the same words). The
-// last wave to finish resets the quad counter for the next launch.
+// Persistent draw: each wave takes 8x8 pixel quads (numbered row by row), lane l
+// drawing pixel (l & 7, l >> 3) of the quad. Chunk masks go to per-lane LDS rows on
+// chunk entry; the chunk-grid occupancy bits are read through L2 (neighbouring primary
+// rays read the same words). Bound by the latency of the walks' loads. Waves per SIMD:
+// without transparent voxels 6 (80 VGPRs; 1920x1080 over 512x256x512 voxels 226 us, 238
+// without the finite-delta walk; 5 waves 235, 7 270, 8 253, 4 242), with them 4 (126).
 #ifndef DN_DRAW_WAVES
-#define DN_DRAW_WAVES 4
+#define DN_DRAW_WAVES 6
 #endif
 template <bool OPAQUE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DN_DRAW_WAVES, DN_DRAW_WAVES)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OPAQUE ? DN_DRAW_WAVES : 4, OPAQUE ? DN_DRAW_WAVES : 4)))
 void k_draw(DNdrawParams P)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -202,11 +205,11 @@ namespace {
 
 // Waves per SIMD the lighting kernel is compiled for, without and with transparent
 // voxels (512x256x512 voxels, every exposed chunk lit; 296x104x232 with glass and
-// mirrors, two samples). Opaque: 3 waves (131 VGPRs) 972 us, 4 (127) 1030, 2 912 but
-// 610 against 530 us in the batch of 24 volumes. General: 5 (96 VGPRs and some 110
-// spilled, outside the walks) 4440 us, 4 (128) 5560, 6 4560, 8 5120.
+// mirrors, two samples). Opaque: 4 waves (128 VGPRs) 403 us, 3 490, 5 583, 6 725; the
+// batch of 24 volumes 327, 355, 362, 397. General: 5 (96 VGPRs and some 110 spilled,
+// outside the walks) 4150 us, 4 (128) 4870, 6 4170.
 #ifndef DN_LIGHT_WAVES
-#define DN_LIGHT_WAVES 3
+#define DN_LIGHT_WAVES 4
 #endif
 #ifndef DN_LIGHT_GENERAL_WAVES
 #define DN_LIGHT_GENERAL_WAVES 5
@@ -238,8 +241,8 @@ void k_lighting(DNlightParams P)
         __syncthreads();
         sv.occLoaded = occLds;
     }
-    // A unit: the voxels of two requests. Four units at a time: 775 us against 951
-    // where every exposed chunk of 512x256x512 voxels is lit (one atomic in 7 is left);
+    // A unit: the voxels of two requests. Four units at a time, all of one line: 775 us
+    // against 951 where every exposed chunk of 512x256x512 voxels is lit;
     // not with specular materials, whose voxels trace up to 15 times the rays of others
     // (296x104x232 with mirrors: 7100 against 4840 us).
     WaveUnits work(P.workCounter + WORK_LIGHT, (nreq + 1u) / 2u, P.copyBack == 0u);
@@ -266,14 +269,14 @@ void k_lighting(DNlightParams P)
 // with the term (the pass adds them whenever it uses it), so the pass's counts
 // are those of tracing in sequence. Voxels without a diffuse term (specular
 // >= 1) are skipped. A wave takes one request (32 slots) at a time.
-// Waves per SIMD the direct-ray kernel is compiled for: 5 (81 VGPRs without and 96
-// with transparent voxels, no spills). Every exposed chunk of 512x256x512 voxels, 32
-// directions, opaque: 5 waves 2120 us, 6 2080, 7 2130; the camera's chunks of a 128^3
-// map: 178, 187, 202.
+// Waves per SIMD the direct-ray kernel is compiled for: 6 without transparent voxels
+// (80 VGPRs), 5 with (96). Every exposed chunk of 512x256x512 voxels, 32 directions,
+// opaque: 6 waves 1835 us, 5 1945, 7 1862, 8 2300; the camera's chunks of a 128^3 map
+// 65, 65, 80, 82.
 // The chunk-grid occupancy bitmap is read from L2 here: staging it in LDS
 // (16 KiB per block on that map) would hold the kernel to 4 waves.
 #ifndef DN_DIRECT_WAVES
-#define DN_DIRECT_WAVES 5
+#define DN_DIRECT_WAVES 6
 #endif
 // The batched direct pass (384 uneven volumes, 16 directions: 4 voxels per
 // wave) measured 49.0 ms of graph time at 6 waves against 52.0 at 5 (with the
@@ -374,7 +377,7 @@ __device__ __forceinline__ void direct_request(const DNlightParams& P, const DNs
 }
 
 template <bool OPAQUE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DN_DIRECT_WAVES, DN_DIRECT_WAVES)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OPAQUE ? DN_DIRECT_WAVES : 5, OPAQUE ? DN_DIRECT_WAVES : 5)))
 void k_direct(DNlightParams P)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -633,21 +636,35 @@ __global__ __launch_bounds__(256) void k_upload(uint32_t* flags, uint32_t* lastU
 }
 
 // ---------------------------------------------------------------------------
-// ray batch: one step_map per ray
+// ray batch
 
 struct RayHit { uint32_t hit, voxelIndex, mapSteps, voxelSteps; float pos[3]; float normal[3]; };
 
-__global__ __launch_bounds__(256) void k_rays(DNrayParams P)
+// Rays of a batch have nothing in common, so a wave's lanes spread over walks of very
+// different length. Without transparent voxels each takes the two nested walks, the
+// wave's lanes entering their chunks together (TOGETHER): 2 000 003 rays over
+// 256x128x256 voxels 394 us at 4 waves per SIMD, 524 without, 297 at 8 (304 with
+// finite deltas told apart). With them, the two walks in one loop.
+template <bool OPAQUE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OPAQUE ? 8 : 6, OPAQUE ? 8 : 6)))
+void k_rays(DNrayParams P)
 {
+    __shared__ uint32_t maskRows[OPAQUE ? DN_MASK_LDS_WORDS(256) : 1];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     RayCtx c;
     ctx_init(c);
+    if(OPAQUE) c.maskRow = lane_mask_row(maskRows);
     if(i < P.n)
     {
         f3 dir = ld3(P.dirs + 3 * (size_t)i), p = ld3(P.origins + 3 * (size_t)i), nrm = splat(0.0f), ca;
         float cm;
         DVoxel vox = {};
-        bool h = step_map_flat<true>(P.scene, c, dir, vinv(dir), p, P.ignoreFirst != 0, vox, ca, cm, nrm);
+        bool h;
+        if constexpr(OPAQUE)
+            h = step_map<false, true, false, true, true>(P.scene, c, dir, vinv(dir), p, P.ignoreFirst != 0, nrm, vox, ca,
+                                                         cm);
+        else
+            h = step_map_flat<true>(P.scene, c, dir, vinv(dir), p, P.ignoreFirst != 0, vox, ca, cm, nrm);
         RayHit o;
         o.hit = h ? 1u : 0u;
         o.voxelIndex = h ? c.hitIndex : 0xFFFFFFFFu;
@@ -974,7 +991,7 @@ int dn_launch_upload(uint32_t* flags, uint32_t* lastUsed, DNchunkRec* chunks, ui
 int dn_launch_rays(const DNrayParams& p, hipStream_t stream)
 {
     if(p.n == 0) return 0;
-    hipLaunchKernelGGL(k_rays, dim3((p.n + 255) / 256), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(p.scene.opaque ? k_rays<true> : k_rays<false>, dim3((p.n + 255) / 256), dim3(256), 0, stream, p);
     return (int)hipGetLastError();
 }
 

@@ -117,3 +117,27 @@ def test_direct_rays_in_parts_of_requests(gpu, n_direct, visible):
     batch.close()
     for v in vols:
         v.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 257, 4099])
+def test_ray_batches_against_oracle(gpu, n):
+    """Rays that start anywhere, outside the map too."""
+    sc = scenes.config_small(seed=23)
+    vol = load_scene(sc)
+    rng = np.random.default_rng(n)
+    org = ((rng.random((n, 3)) * 1.2 - 0.1) * sc.map_size).astype(np.float32)
+    d = (rng.standard_normal((n, 3)) + 1e-4).astype(np.float32)
+    o = oracle.load("f32")
+    s, _ = oracle_scene(o, vol, sc)
+    vol.counters(2, reset=True)
+    for first in (False, True):
+        r = vol.cast_rays(org, d, first)
+        want, _ = o.cast_rays(s, org, d, ignore_first=first)
+        for f in ("hit", "voxelIndex", "mapSteps", "voxelSteps"):
+            assert np.array_equal(r[f], want[f]), f
+        assert np.array_equal(r["pos"].view(np.uint32), want["pos"].view(np.uint32))
+        assert np.array_equal(r["normal"].view(np.uint32) & 0x7FFFFFFF, want["normal"].view(np.uint32) & 0x7FFFFFFF)
+        c = vol.counters(2, reset=True)
+        assert c["rays"] == n and c["hits"] == int(want["hit"].sum())
+        assert c["mapSteps"] == int(want["mapSteps"].sum()) and c["voxelSteps"] == int(want["voxelSteps"].sum())
+    vol.close()
