@@ -762,23 +762,36 @@ __device__ __forceinline__ float ema_one(float& e, float w, const DNrcAdam& o)
     return e * o.emaScale;
 }
 
-__global__ __launch_bounds__(256) void k_rc_adam(DNrcNet net, DNrcAdam o, size_t entries)
+// A dense level's table ends in entries that no corner has: they are never read, and
+// their gradients and moments stay zero, so the step leaves them as they are (45% of
+// the table at 2^19 entries and resolutions 16..256). `used`: the entries of a level
+// that the step covers, in whole blocks of 256.
+struct DNrcUsed { uint32_t blocks[RC_LEVELS + 1]; };     // first block of each level, and their number
+
+// 44 bytes a parameter: bound by HBM.
+__global__ __launch_bounds__(256) void k_rc_adam(DNrcNet net, DNrcAdam o, DNrcUsed used)
 {
-    const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
-    if(i < RC_NPARAM)
+    if(blockIdx.x < RC_NPARAM / 256u)
     {
+        const uint32_t i = blockIdx.x * 256u + threadIdx.x;
         float w = net.w32[i], m = net.wM[i], v = net.wV[i], e = net.wE[i];
         adam_one(w, net.wGrad[i], m, v, o);
         net.w32[i] = w; net.wM[i] = m; net.wV[i] = v;
         net.wGrad[i] = 0.0f;
         uint32_t f, t;
-        rc_fragment_positions((uint32_t)i, f, t);
+        rc_fragment_positions(i, f, t);
         net.w16[f] = net.wT16[t] = f2bf(w);
         net.wE16[f] = f2bf(ema_one(e, w, o));
         net.wE[i] = e;
     }
-    if(i < entries)
+    else
     {
+        const uint32_t b = blockIdx.x - RC_NPARAM / 256u;
+        uint32_t l = 0;
+        for(uint32_t k = 1; k < RC_LEVELS; k++) l += b >= used.blocks[k] ? 1u : 0u;
+        const uint32_t in = (b - used.blocks[l]) * 256u + threadIdx.x;
+        if(in >> net.log2T) return;                      // tables smaller than a block
+        const size_t i = ((size_t)l << net.log2T) + in;
         float2 w = reinterpret_cast<float2*>(net.tab32)[i];
         float2 g = reinterpret_cast<float2*>(net.tabGrad)[i];
         float2 m = reinterpret_cast<float2*>(net.tabM)[i];
@@ -1134,9 +1147,18 @@ int dn_rc_train(const DNrcNet& net, const float* samples, uint32_t n, const DNrc
 
 int dn_rc_adam(const DNrcNet& net, const DNrcAdam& opt, hipStream_t stream)
 {
-    const size_t entries = (size_t)RC_LEVELS << net.log2T;
-    hipLaunchKernelGGL(k_rc_adam, dim3(blocks_for(entries > RC_NPARAM ? entries : RC_NPARAM)), dim3(256), 0, stream,
-                       net, opt, entries);
+    // with moments of zero a step adds +-0 to a parameter, unless it divides by zero
+    const bool skip = opt.bias1 > 0.0f && opt.bias2 > 0.0f && opt.eps > 0.0f && opt.lr >= 0.0f &&
+                      opt.lr < INFINITY;
+    DNrcUsed used;
+    used.blocks[0] = 0;
+    for(uint32_t l = 0; l < RC_LEVELS; l++)
+    {
+        const uint64_t S = net.res[l] + 2ull, T = 1ull << net.log2T;
+        const uint64_t entries = skip && ((net.denseMask >> l) & 1u) ? S * S * S : T;
+        used.blocks[l + 1] = used.blocks[l] + (uint32_t)((entries + 255u) / 256u);
+    }
+    hipLaunchKernelGGL(k_rc_adam, dim3(RC_NPARAM / 256u + used.blocks[RC_LEVELS]), dim3(256), 0, stream, net, opt, used);
     return (int)hipGetLastError();
 }
 
