@@ -73,14 +73,9 @@ struct DNrcNet {
     float* wE;
     uint16_t* wE16;
 };
-// Per-batch activation buffers of training, `tiles` = samples / 16. The *T
-// buffers are tile-transposed bf16: [tile][feature][16 samples].
+// Per-batch buffers of training.
 struct DNrcActs {
     uint32_t* x0;                  // [RC_LEVELS][samples] a level's two bf16 features
-    uint16_t* x0T;                 // [tile][48][16]
-    uint16_t* hT[3];               // [tile][64][16]
-    uint16_t* dzT[3];              // [tile][64][16]
-    uint16_t* dyT;                 // [tile][16][16]
     float* denc;                   // [RC_LEVELS][samples][2] gradients of the encoded features
     // Table gradients by bucket (rc_bucketed): positions over the extent, the
     // records of every level, bucket and sorting block, those of every level and
@@ -104,8 +99,9 @@ struct DNrcAdam {
 
 // pred: float4 per row (3 outputs plus the row's exact term, the row's valid flag).
 int dn_rc_predict(const DNrcNet& net, const float* samples, uint32_t n, float* pred, hipStream_t stream);
-// A second stream for training: the weight gradients run on it beside the
-// table gradients (`fork` and `join` order it after the MLP and before Adam).
+// A second stream for training: the corner rows are sorted on it beside the encoding
+// and the MLP (`fork` and `join` order it after what came before and before the table
+// gradients).
 struct DNrcSide {
     hipStream_t stream;
     hipEvent_t fork, join;

@@ -111,12 +111,8 @@ bool ensure_train(DNXradianceCache* rc, uint32_t n)
     if(n <= rc->cap) return true;
     DNrcActs& a = rc->acts;
     hipStreamSynchronize(rc->stream);
-    dfree(a.x0); dfree(a.x0T); dfree(a.dyT); dfree(a.denc); dfree(a.unit); dfree(a.records);
-    for(int i = 0; i < 3; i++) { dfree(a.hT[i]); dfree(a.dzT[i]); }
-    bool g = dev(&a.x0, (size_t)n * RC_LEVELS, "activations") && dev(&a.x0T, (size_t)n * RC_IN, "activations") &&
-             dev(&a.dyT, (size_t)n * RC_OUT, "activations") && dev(&a.denc, (size_t)n * RC_ENC, "activations");
-    for(int i = 0; g && i < 3; i++)
-        g = dev(&a.hT[i], (size_t)n * RC_W, "activations") && dev(&a.dzT[i], (size_t)n * RC_W, "activations");
+    dfree(a.x0); dfree(a.denc); dfree(a.unit); dfree(a.records);
+    bool g = dev(&a.x0, (size_t)n * RC_LEVELS, "activations") && dev(&a.denc, (size_t)n * RC_ENC, "activations");
     const uint32_t most = std::min(n, (uint32_t)RC_BUCKETED_MAX);      // later, smaller calls may be bucketed
     if(rc_bucketed(rc->net, most))
     {
@@ -222,9 +218,8 @@ extern "C" void DNX_rc_destroy(DNXradianceCache* rc)
     dfree(n.tab16); dfree(n.tab32); dfree(n.tabGrad); dfree(n.tabM); dfree(n.tabV); dfree(n.tabE); dfree(n.tabE16);
     dfree(n.w16); dfree(n.wT16); dfree(n.w32); dfree(n.wGrad); dfree(n.wM); dfree(n.wV); dfree(n.wE); dfree(n.wE16);
     DNrcActs& a = rc->acts;
-    dfree(rc->dSamples); dfree(a.x0); dfree(a.x0T); dfree(a.dyT); dfree(a.denc);
+    dfree(rc->dSamples); dfree(a.x0); dfree(a.denc);
     dfree(a.unit); dfree(a.records); dfree(a.bucketCount); dfree(a.blockCount);
-    for(int i = 0; i < 3; i++) { dfree(a.hT[i]); dfree(a.dzT[i]); }
     dfree(rc->dQuery);
     delete rc;
 }

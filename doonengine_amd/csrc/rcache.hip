@@ -7,14 +7,13 @@
 // (x * 1 ^ y * 2654435761 ^ z * 805459861) mod T.
 // Network: 4 weight matrices without biases, ReLU between them; operands in
 // bfloat16 on v_mfma_f32_16x16x32_bf16 (v_mfma_f32_16x16x16_bf16 for a
-// lone 16-wide K block and for the weight-gradient GEMM) with FP32
-// accumulation. Layers are
+// lone 16-wide K block) with FP32 accumulation. Layers are
 // computed transposed (D[feature][sample] = W * X^T), so one layer's 16x16
 // accumulator tile is, lane for lane, the next layer's B operand: a lane holds
 // sample (lane & 15) and features 4 * (lane >> 4) + 0..3 of a 16-feature block.
-// Training: forward + backward per 16-sample tile, weight gradients as a
-// split-K MFMA reduction over the tiles, hash-table gradients by FP32 atomics,
-// then Adam (Kingma & Ba 2015, algorithm 1) on FP32 master copies.
+// Training: forward, backward and the weight gradients (an MFMA product over
+// the samples) in one kernel, hash-table gradients by FP32 atomics or summed in
+// LDS by bucket, then Adam (Kingma & Ba 2015, algorithm 1) on FP32 master copies.
 #include "dn_light.hpp"
 #include "rc_internal.h"
 #include "doon/doon.h"
@@ -86,17 +85,6 @@ __device__ __forceinline__ bf16x4 relu_grad(f32x4 d, bf16x4 h)
 {
     for(int i = 0; i < 4; i++) d[i] = h[i] > 0 ? d[i] : 0.0f;     // bits of h: not -0, +0 or negative
     return to_bf16(d);
-}
-
-// Stores a C-layout bf16 tile of feature block fb into a tile-transposed
-// buffer T[tile][F][16].
-__device__ __forceinline__ void store_T(uint16_t* T, uint32_t F, uint32_t tile, uint32_t fb, bf16x4 v, uint32_t lane)
-{
-    uint16_t* p = T + ((size_t)tile * F + fb * 16u + 4u * (lane >> 4)) * 16u + (lane & 15u);
-    p[0] = (uint16_t)v[0];
-    p[16] = (uint16_t)v[1];
-    p[32] = (uint16_t)v[2];
-    p[48] = (uint16_t)v[3];
 }
 
 // ---------------------------------------------------------------------------
@@ -633,44 +621,107 @@ __global__ __launch_bounds__(256) void k_rc_predict(DNrcNet net, const float* sa
     }
 }
 
-// Forward and backward of training, one tile per wave at a time.
-__global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const float* samples, uint32_t n, float invB,
-                                                DNrcActs acts)
+// Forward, backward and weight gradients of training: one tile per wave at a time, the
+// RC_MLP_WAVES tiles of a block together for the weight gradients dW = dZ^T X, whose K
+// is the samples. Layer by layer the block's dZ and X go to LDS as [feature][sample]
+// and each wave multiplies its six 16x16 tiles of the 48 (v_mfma_f32_16x16x32_bf16,
+// 32 samples a step), so a wave holds 24 accumulators over all its tiles and neither
+// activations nor dZ go to memory: 900 bytes a sample, which a launch of its own used
+// to read back (2^17 samples: 41 us against 41 and 47, and 139 where that launch ran
+// beside the table gradients).
+#define RC_MLP_WAVES 8
+// One block a CU (210 VGPRs, 80 KiB of LDS): 41 us per 2^17 samples beside the sorting
+// kernels, 69 at 512 blocks.
+#define RC_MLP_BLOCKS 256u
+enum { RC_SPAN = 16 * RC_MLP_WAVES };          // samples of a block's tiles
+
+// Position in a staged matrix of sample s of feature f: rows of RC_SPAN samples, whose
+// 16-byte pieces (8 samples) are permuted by the feature, so that 16 lanes which read
+// the same piece of 16 rows meet all banks.
+__device__ __forceinline__ uint32_t staged_at(uint32_t f, uint32_t s)
 {
+    return f * RC_SPAN + (((s >> 3) ^ (f & (RC_SPAN / 8u - 1u))) << 3) + (s & 7u);
+}
+
+// Writes a C-layout tile of feature block fb: sample `s` of the block's, features
+// 16 fb + 4 q + 0..3.
+__device__ __forceinline__ void stage_tile(uint16_t* m, uint32_t fb, uint32_t q, uint32_t s, bf16x4 v)
+{
+    #pragma unroll
+    for(uint32_t i = 0; i < 4u; i++) m[staged_at(16u * fb + 4u * q + i, s)] = (uint16_t)v[i];
+}
+
+// acc += A B^T over the block's samples: 16 rows of each of two staged matrices.
+__device__ __forceinline__ f32x4 samples_product(const uint16_t* a, uint32_t ab, const uint16_t* b, uint32_t bb,
+                                                 uint32_t lane, f32x4 acc)
+{
+    const uint32_t r = lane & 15u, q = lane >> 4;
+    #pragma unroll
+    for(uint32_t k = 0; k < RC_SPAN; k += 32u)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(a + staged_at(16u * ab + r, k + 8u * q))),
+            __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(b + staged_at(16u * bb + r, k + 8u * q))), acc, 0,
+            0, 0);
+    return acc;
+}
+
+// Adds a C-layout tile of a weight gradient: rows 16 rb + 4 q + 0..3, column 16 cb + lane mod 16.
+__device__ __forceinline__ void add_wgrad(float* g, uint32_t ld, uint32_t rb, uint32_t cb, uint32_t lane, f32x4 v)
+{
+    for(uint32_t i = 0; i < 4u; i++)
+        atomicAdd(g + (16u * rb + 4u * (lane >> 4) + i) * ld + 16u * cb + (lane & 15u), v[i]);
+}
+
+__global__ __launch_bounds__(64 * RC_MLP_WAVES) void k_rc_mlp(DNrcNet net, const float* samples, uint32_t n,
+                                                              float invB, DNrcActs acts)
+{
+    static_assert(RC_MLP_WAVES == 8, "six tiles of the weight gradients per wave");
     __shared__ __align__(16) uint16_t W[RC_NPARAM];
     __shared__ __align__(16) uint16_t WT[RC_NPARAM];
-    stage_weights(W, net.w16, 256u);
-    stage_weights(WT, net.wT16, 256u);
+    __shared__ __align__(16) uint16_t Z[RC_W * RC_SPAN];
+    __shared__ __align__(16) uint16_t X[RC_W * RC_SPAN];
+    stage_weights(W, net.w16, 64u * RC_MLP_WAVES);
+    stage_weights(WT, net.wT16, 64u * RC_MLP_WAVES);
     __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u, q = lane >> 4;
-    const uint32_t tiles = n / 16u;
+    const uint32_t lane = threadIdx.x & 63u, q = lane >> 4, w = threadIdx.x >> 6;
+    const uint32_t tiles = n / 16u, at = w * 16u + (lane & 15u);
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    for(uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6); tile < tiles; tile += gridDim.x * 4u)
+    // this wave's tiles: rows w / 2, columns 2 (w mod 2) and the next of W1 and W2; of
+    // W0's 4 x 3, waves 0..3 two and waves 4..7 one; of W3's four, waves 4..7 one
+    f32x4 g1[2] = {zero, zero}, g2[2] = {zero, zero}, g0a = zero, gb = zero;
+    for(uint32_t base = blockIdx.x * RC_MLP_WAVES; base < tiles; base += gridDim.x * RC_MLP_WAVES)
     {
-        const uint32_t sm = tile * 16u + (lane & 15u);
+        const uint32_t tile = base + w;
+        const bool on = tile < tiles;                   // waves past the end take a tile without weight
+        const uint32_t sm = (on ? tile : tiles - 1u) * 16u + (lane & 15u);
         const float* row = samples + (size_t)sm * RC_SAMPLE;
         bf16x4 xin[3], h[3][4];
         f32x4 y;
         load_input(acts.x0, n, sm, row, q, xin);
         mlp_forward(W, lane, xin, h, y);
-        for(uint32_t ks = 0; ks < 3; ks++) store_T(acts.x0T, RC_IN, tile, ks, xin[ks], lane);
-        for(uint32_t layer = 0; layer < 3; layer++)
-            for(uint32_t mb = 0; mb < 4; mb++) store_T(acts.hT[layer], RC_W, tile, mb, h[layer][mb], lane);
         // dL/dy = (y - t) / B for valid samples
         f32x4 dy = zero;
-        if(lane < 16u && row[12] != 0.0f)
+        if(on && lane < 16u && row[12] != 0.0f)
             for(int i = 0; i < 3; i++) dy[i] = (y[i] - row[9 + i]) * invB;
         const bf16x4 dyb = to_bf16(dy);
-        store_T(acts.dyT, RC_OUT, tile, 0, dyb, lane);
+        __syncthreads();                                // the tiles before are multiplied
+        stage_tile(Z, 0, q, at, dyb);
+        for(uint32_t mb = 0; mb < 4; mb++) stage_tile(X, mb, q, at, h[2][mb]);
         // dH3^T = W3^T dY^T (K = 16 outputs), then through the ReLUs
         bf16x4 dz[4];
         for(uint32_t mb = 0; mb < 4; mb++)
-        {
             dz[mb] = relu_grad(mfma16(a_frag16(WT + RC_OFF_W3 + mb * 256u, lane), dyb, zero), h[2][mb]);
-            store_T(acts.dzT[2], RC_W, tile, mb, dz[mb], lane);
-        }
+        __syncthreads();
+        if(w >= 4u) gb = samples_product(Z, 0, X, w - 4u, lane, gb);
+        #pragma unroll
         for(int layer = 1; layer >= 0; layer--)
         {
+            __syncthreads();
+            for(uint32_t mb = 0; mb < 4; mb++)
+            {
+                stage_tile(Z, mb, q, at, dz[mb]);
+                stage_tile(X, mb, q, at, h[layer][mb]);
+            }
             // dH_layer^T = W_{layer+1}^T dZ_{layer+1}^T
             const uint16_t* WTl = WT + (layer == 1 ? RC_OFF_W2 : RC_OFF_W1);
             bf16x4 nz[4];
@@ -679,10 +730,18 @@ __global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const float* sample
                 f32x4 d = mfma32(a_frag32(WTl + mb * 1024u, lane), dz[0], dz[1], zero);
                 d = mfma32(a_frag32(WTl + mb * 1024u + 512u, lane), dz[2], dz[3], d);
                 nz[mb] = relu_grad(d, h[layer][mb]);
-                store_T(acts.dzT[layer], RC_W, tile, mb, nz[mb], lane);
+            }
+            __syncthreads();
+            for(uint32_t k = 0; k < 2u; k++)
+            {
+                f32x4& g = layer == 1 ? g2[k] : g1[k];
+                g = samples_product(Z, w >> 1, X, 2u * (w & 1u) + k, lane, g);
             }
             for(uint32_t mb = 0; mb < 4; mb++) dz[mb] = nz[mb];
         }
+        __syncthreads();
+        for(uint32_t mb = 0; mb < 4; mb++) stage_tile(Z, mb, q, at, dz[mb]);
+        for(uint32_t ks = 0; ks < 3; ks++) stage_tile(X, ks, q, at, xin[ks]);
         // dX0^T = W0^T dZ1^T, encoded features only (rows 0..31)
         for(uint32_t mb = 0; mb < 2; mb++)
         {
@@ -690,59 +749,24 @@ __global__ __launch_bounds__(256) void k_rc_mlp(DNrcNet net, const float* sample
             d = mfma32(a_frag32(WT + RC_OFF_W0 + mb * 1024u + 512u, lane), dz[2], dz[3], d);
             // features 16 mb + 4 q + 0..3: levels 8 mb + 2 q and the next
             float2* g = reinterpret_cast<float2*>(acts.denc) + (size_t)(8u * mb + 2u * q) * n + sm;
-            g[0] = make_float2(d[0], d[1]);
-            g[n] = make_float2(d[2], d[3]);
+            if(on)
+            {
+                g[0] = make_float2(d[0], d[1]);
+                g[n] = make_float2(d[2], d[3]);
+            }
         }
+        __syncthreads();
+        g0a = samples_product(Z, w & 3u, X, w < 4u ? 0u : 2u, lane, g0a);
+        if(w < 4u) gb = samples_product(Z, w, X, 1u, lane, gb);
     }
-}
-
-// Weight gradients dW = dZ^T X summed over all tiles (K = samples, one
-// 16-sample tile per v_mfma_f32_16x16x16_bf16: pairing two tiles into one
-// K = 32 step doubles the scattered 8-byte operand loads per step and measured
-// 153 against 69 us per 2^17 samples at 128 blocks); blocks take contiguous tile ranges; wave w owns output rows 16w..16w+15 of W0..W2 and output
-// column block w of W3; partial sums go out by FP32 atomics.
-__global__ __launch_bounds__(256) void k_rc_wgrad(DNrcNet net, uint32_t tiles, DNrcActs acts)
-{
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    const uint32_t per = (tiles + gridDim.x - 1u) / gridDim.x;
-    const uint32_t t0 = blockIdx.x * per, t1 = min(tiles, t0 + per);
-    f32x4 a0[3], a1[4], a2[4], a3;
-    for(int i = 0; i < 3; i++) a0[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for(int i = 0; i < 4; i++) { a1[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f}; a2[i] = a1[i]; }
-    a3 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t row = w * 16u + (lane & 15u);           // A rows: output features
-    const uint32_t kq = 4u * (lane >> 4);                  // samples 4*(lane>>4)..+3 of the tile
-    for(uint32_t t = t0; t < t1; t++)
+    if(blockIdx.x * RC_MLP_WAVES >= tiles) return;
+    add_wgrad(net.wGrad + RC_OFF_W0, 48u, w & 3u, w < 4u ? 0u : 2u, lane, g0a);
+    if(w < 4u) add_wgrad(net.wGrad + RC_OFF_W0, 48u, w, 1u, lane, gb);
+    else add_wgrad(net.wGrad + RC_OFF_W3, 64u, 0u, w - 4u, lane, gb);
+    for(uint32_t k = 0; k < 2u; k++)
     {
-        const size_t b64 = (size_t)t * RC_W * 16u, b48 = (size_t)t * RC_IN * 16u, b16 = (size_t)t * RC_OUT * 16u;
-        bf16x4 A0 = ld_bf16x4(acts.dzT[0] + b64 + row * 16u + kq);
-        bf16x4 A1 = ld_bf16x4(acts.dzT[1] + b64 + row * 16u + kq);
-        bf16x4 A2 = ld_bf16x4(acts.dzT[2] + b64 + row * 16u + kq);
-        for(uint32_t nb = 0; nb < 3; nb++)
-            a0[nb] = mfma16(A0, ld_bf16x4(acts.x0T + b48 + (nb * 16u + (lane & 15u)) * 16u + kq), a0[nb]);
-        for(uint32_t nb = 0; nb < 4; nb++)
-        {
-            const uint32_t col = (nb * 16u + (lane & 15u)) * 16u + kq;
-            a1[nb] = mfma16(A1, ld_bf16x4(acts.hT[0] + b64 + col), a1[nb]);
-            a2[nb] = mfma16(A2, ld_bf16x4(acts.hT[1] + b64 + col), a2[nb]);
-        }
-        bf16x4 A3 = ld_bf16x4(acts.dyT + b16 + (lane & 15u) * 16u + kq);
-        a3 = mfma16(A3, ld_bf16x4(acts.hT[2] + b64 + (w * 16u + (lane & 15u)) * 16u + kq), a3);
-    }
-    if(t0 >= t1) return;
-    // C layout: column (input feature) nb*16 + (lane & 15), rows 16w + 4*(lane>>4) + i
-    const uint32_t r0 = w * 16u + 4u * (lane >> 4);
-    for(uint32_t i = 0; i < 4; i++)
-    {
-        for(uint32_t nb = 0; nb < 3; nb++)
-            atomicAdd(net.wGrad + RC_OFF_W0 + (r0 + i) * 48u + nb * 16u + (lane & 15u), a0[nb][i]);
-        for(uint32_t nb = 0; nb < 4; nb++)
-        {
-            atomicAdd(net.wGrad + RC_OFF_W1 + (r0 + i) * 64u + nb * 16u + (lane & 15u), a1[nb][i]);
-            atomicAdd(net.wGrad + RC_OFF_W2 + (r0 + i) * 64u + nb * 16u + (lane & 15u), a2[nb][i]);
-        }
-        // W3: rows = outputs 4*(lane>>4) + i, column block w
-        atomicAdd(net.wGrad + RC_OFF_W3 + (4u * (lane >> 4) + i) * 64u + w * 16u + (lane & 15u), a3[i]);
+        add_wgrad(net.wGrad + RC_OFF_W1, 64u, w >> 1, 2u * (w & 1u) + k, lane, g1[k]);
+        add_wgrad(net.wGrad + RC_OFF_W2, 64u, w >> 1, 2u * (w & 1u) + k, lane, g2[k]);
     }
 }
 
@@ -1093,32 +1117,32 @@ int dn_rc_train(const DNrcNet& net, const float* samples, uint32_t n, const DNrc
     if(n == 0 || (n & 15u)) return n ? (int)hipErrorInvalidValue : 0;
     const uint32_t tiles = n / 16u;
     const bool bucketed = rc_bucketed(net, n);
-    hipLaunchKernelGGL(k_rc_encode, dim3(8u * blocks_for(n)), dim3(256), 0, stream, net, samples, n, a.x0);
-    if(bucketed)
-    {
-        const uint32_t chunks = (n + 4095u) / 4096u;
-        const dim3 grid(chunks < RC_SORT_BLOCKS ? chunks : (uint32_t)RC_SORT_BLOCKS, RC_LEVELS);
-        hipLaunchKernelGGL(k_rc_bucket_count, grid, dim3(1024), 0, stream, net, samples, n, a);
-        hipLaunchKernelGGL(k_rc_bucket_place, grid, dim3(1024), 0, stream, net, n, a);
-    }
-    // at most 512 blocks (4 tiles per wave at 2^17 samples): 83 us per 2^17 samples against 92 at
-    // 1024 blocks, 98 at 256 and 82 at 768
-    hipLaunchKernelGGL(k_rc_mlp, dim3(blocks_for((size_t)tiles * 64u, 512)), dim3(256), 0, stream, net, samples, n,
-                       1.0f / (float)n, a);
-    // The weight gradients (MFMA and LDS bound) and the table gradients (bound
-    // by their atomics) read the same activations and write disjoint buffers:
-    // with a side stream they run side by side.
-    // one block per CU (47 us per 2^17 samples; 128 blocks 71 us, 512 blocks 50 us)
-    const uint32_t wb = tiles < 256u ? tiles : 256u;
-    hipStream_t ws = stream;
-    if(side)
+    // The corner rows are sorted (bound by LDS atomics) beside the encoding (bound by
+    // its gathers) and the MLP: they share nothing but the samples. (Sorting the next
+    // step's rows beside this step's table gradients and Adam: 2371 against 2275 us per
+    // 8 steps of 2^17 rows; the gradients then wait for LDS.)
+    hipStream_t ss = stream;
+    if(bucketed && side)
     {
         if(hipEventRecord(side->fork, stream) != hipSuccess ||
            hipStreamWaitEvent(side->stream, side->fork, 0) != hipSuccess)
             return (int)hipErrorLaunchFailure;
-        ws = side->stream;
+        ss = side->stream;
     }
-    hipLaunchKernelGGL(k_rc_wgrad, dim3(wb), dim3(256), 0, ws, net, tiles, a);
+    if(bucketed)
+    {
+        const uint32_t chunks = (n + 4095u) / 4096u;
+        const dim3 grid(chunks < RC_SORT_BLOCKS ? chunks : (uint32_t)RC_SORT_BLOCKS, RC_LEVELS);
+        hipLaunchKernelGGL(k_rc_bucket_count, grid, dim3(1024), 0, ss, net, samples, n, a);
+        hipLaunchKernelGGL(k_rc_bucket_place, grid, dim3(1024), 0, ss, net, n, a);
+    }
+    hipLaunchKernelGGL(k_rc_encode, dim3(8u * blocks_for(n)), dim3(256), 0, stream, net, samples, n, a.x0);
+    const uint32_t spans = (tiles + RC_MLP_WAVES - 1u) / RC_MLP_WAVES;
+    hipLaunchKernelGGL(k_rc_mlp, dim3(spans < RC_MLP_BLOCKS ? spans : RC_MLP_BLOCKS), dim3(64u * RC_MLP_WAVES), 0,
+                       stream, net, samples, n, 1.0f / (float)n, a);
+    if(bucketed && side && (hipEventRecord(side->join, side->stream) != hipSuccess ||
+                            hipStreamWaitEvent(stream, side->join, 0) != hipSuccess))
+        return (int)hipErrorLaunchFailure;
     if(bucketed)
     {
         // blocks take several slices where there are more than two per CU (all can be
@@ -1139,9 +1163,6 @@ int dn_rc_train(const DNrcNet& net, const float* samples, uint32_t n, const DNrc
         // one wave per 16 samples and level
         hipLaunchKernelGGL(k_rc_table_grad, dim3(blocks_for((size_t)RC_LEVELS * ((n + 15u) / 16u) * 64u)), dim3(256), 0,
                        stream, net, samples, n, (const float*)a.denc);
-    if(side && (hipEventRecord(side->join, side->stream) != hipSuccess ||
-                hipStreamWaitEvent(stream, side->join, 0) != hipSuccess))
-        return (int)hipErrorLaunchFailure;
     return (int)hipGetLastError();
 }
 

@@ -9,7 +9,7 @@ import pytest
 
 from doonengine_amd import scenes
 from doonengine_amd._hip import DeviceBuffer
-from doonengine_amd.volume import RadianceCache, Volume, rc_pack_weights
+from doonengine_amd.volume import RadianceCache, Volume, rc_pack_weights, rc_unpack_weights
 from oracle import radiance_cache as orc
 
 pytestmark = pytest.mark.gpu
@@ -92,3 +92,31 @@ def test_many_rows_gradients_match_oracle(volume, log2, n, narrow):
     d = ref["dtable"]
     assert np.linalg.norm(tg - d) / np.linalg.norm(d) < 5e-3
     assert np.linalg.norm(twice.reshape(table.shape) - 2.0 * tg) / np.linalg.norm(tg) < 1e-5      # calls add up
+
+
+@pytest.mark.parametrize("n", [16, 112, 128, 144, 2048 + 16, 32768 + 48])
+def test_weight_gradients_at_block_edges(volume, n):
+    """Weight gradients are multiplied per block of eight 16-row tiles: one tile, one
+    short of a block, a block, one more, and more blocks than the grid has. Rows
+    without weight (valid 0) among them."""
+    rng = np.random.default_rng(n)
+    cfg = orc.Config(log2_table=12, extent=EXTENT)
+    mats, table = orc.init_params(cfg, seed=4)
+    table = rng.normal(0, 0.05, table.shape).astype(np.float32)
+    rows = make_rows(rng, n)
+    rows[:, 13:16] = 0.0
+    rc = RadianceCache(volume, log2Table=12, extent=EXTENT, samplesPerFrame=16)
+    try:
+        rc.set_params(rc_pack_weights(mats), table.reshape(-1))
+        rc.train_samples(DeviceBuffer.from_array(rows), n, step=False)
+        g = rc_unpack_weights(rc.get_params()[2])
+        rows[:, 12] = 0.0
+        rc.train_samples(DeviceBuffer.from_array(rows), n, step=False)
+        again = rc_unpack_weights(rc.get_params()[2])
+    finally:
+        rc.close()
+    pos = np.clip(rows[:, 0:3], 0.0, EXTENT)
+    ref = orc.forward_backward(cfg, mats, table, pos, rows[:, 3:6], rows[:, 6:9], rows[:, 9:12], bf16_ops=True)
+    for i, (a, b, c) in enumerate(zip(g, ref["dW"], again)):
+        assert np.linalg.norm(a - b) / np.linalg.norm(b) < 5e-3, i
+        assert np.array_equal(a, c), i
