@@ -136,6 +136,9 @@ __device__ __forceinline__ float corner_weight(const LevelCell& c, uint32_t k)
            ((k & 4u) ? c.f[2] : 1.0f - c.f[2]);
 }
 
+// Two consecutive table entries, which need not start on 8 bytes.
+struct __attribute__((packed, aligned(4))) Pair { uint32_t a, b; };
+
 // A level's two features of a position, as bf16 (first feature in the low half).
 // `level` is the entry index at which the level's table starts. KIND: every lane
 // of the wave is at a dense level (1), at a hashed one (2), or either (0).
@@ -145,18 +148,45 @@ __device__ __forceinline__ uint32_t encode_level(const uint32_t* tab, uint32_t l
 {
     const LevelCell c = level_cell(N, u);
     if(KIND) dense = KIND == 1;
-    // corner (x, y, z): x + y S + z S^2, or x ^ y P ^ z P' mod T
+    // Corner (x, y, z): x + y S + z S^2, or x ^ y P ^ z P' mod T. Bound by the number of
+    // gathers, so a corner and its x neighbour come with one where they lie side by
+    // side: on dense levels always, on hashed ones where x is even (their indices then
+    // differ in the last bit only). 10^6 rows at 2^19 entries: 171 us against 178.
     const uint32_t S = N + 2u;
     const uint32_t my = dense ? S : 2654435761u, mz = dense ? S * S : 805459861u;
     const uint32_t y0 = c.g[1] * my, z0 = c.g[2] * mz;
     uint32_t e[8];
+    uint32_t at[4];
+    Pair p[4];
     #pragma unroll
-    for(uint32_t k = 0; k < 8u; k++)
+    for(uint32_t j = 0; j < 4u; j++)
     {
-        const uint32_t x = c.g[0] + (k & 1u), y = (k & 2u) ? y0 + my : y0, z = (k & 4u) ? z0 + mz : z0;
-        const uint32_t i = (dense ? x + (y + z) : x ^ (y ^ z)) & mask;
+        const uint32_t y = (j & 1u) ? y0 + my : y0, z = (j & 2u) ? z0 + mz : z0;
+        at[j] = dense ? c.g[0] + (y + z) : (c.g[0] ^ (y ^ z)) & mask;
         // a 32-bit byte offset (the tables hold at most 2^28 entries)
-        e[k] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(tab) + ((level + i) << 2));
+        p[j] = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(tab) +
+                                              ((level + (dense ? at[j] : at[j] & ~1u)) << 2));
+    }
+    const bool apart = !dense && (c.g[0] & 1u);
+    uint32_t far[4];
+    #pragma unroll
+    for(uint32_t j = 0; j < 4u; j++) far[j] = 0u;
+    if(apart)
+    {
+        #pragma unroll
+        for(uint32_t j = 0; j < 4u; j++)
+        {
+            const uint32_t y = (j & 1u) ? y0 + my : y0, z = (j & 2u) ? z0 + mz : z0;
+            const uint32_t i = ((c.g[0] + 1u) ^ (y ^ z)) & mask;
+            far[j] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(tab) + ((level + i) << 2));
+        }
+    }
+    #pragma unroll
+    for(uint32_t j = 0; j < 4u; j++)
+    {
+        const bool second = !dense && (at[j] & 1u);
+        e[2 * j] = second ? p[j].b : p[j].a;
+        e[2 * j + 1] = apart ? far[j] : (second ? p[j].a : p[j].b);
     }
     float a0 = 0.0f, a1 = 0.0f;
     #pragma unroll
@@ -573,12 +603,12 @@ __device__ __forceinline__ void mlp_forward(const uint16_t* W, uint32_t lane, co
 
 // Predictions: each lane encodes the four levels whose features it feeds to the
 // first layer, so there is one launch and no pass over encoded rows, and no
-// scratch memory that calls would share. Bound by the 128 table gathers a row
-// needs (2^20 rows: 0.73 T gathers/s where the tables exceed the L2s, 1.05 T/s
-// where they fit). Against encoding all rows in a launch of their own (a level
-// per wave, each XCD two levels) 5.7 against 7.5 us at 1008 rows, 17.6 against
-// 22.6 at 65 536 and 181 against 202 at 10^6 (2^19 entries); one row per
-// 16 lanes with the weights' LDS reads in bank conflict took 13.1, 44.9 and 360.
+// scratch memory that calls would share. Bound by the table gathers (a row's 128
+// corners with some 85 of them; 10^6 rows at 2^19 entries 171 us, 178 with 128).
+// Against encoding all rows in a launch of their own (a level per wave, each XCD two
+// levels), both with 128 gathers, 5.7 against 7.5 us at 1008 rows, 17.6 against 22.6
+// at 65 536 and 181 against 202 at 10^6; one row per 16 lanes with the weights' LDS
+// reads in bank conflict took 13.1, 44.9 and 360.
 __global__ __launch_bounds__(256) void k_rc_predict(DNrcNet net, const float* samples, uint32_t n, float* pred)
 {
     __shared__ __align__(16) uint16_t W[RC_NPARAM];
