@@ -141,3 +141,32 @@ def test_ray_batches_against_oracle(gpu, n):
         assert c["rays"] == n and c["hits"] == int(want["hit"].sum())
         assert c["mapSteps"] == int(want["mapSteps"].sum()) and c["voxelSteps"] == int(want["voxelSteps"].sum())
     vol.close()
+
+
+@pytest.mark.parametrize("split", [1, 3])
+@pytest.mark.parametrize("chunks", [(16, 8, 8), (41, 5, 5), (32, 16, 32), (33, 16, 32)])
+def test_visible_requests_at_launch_edges(gpu, chunks, split):
+    """1024 tiles (one block), one more, the most that one launch takes, and more."""
+    rng = np.random.default_rng(chunks[0])
+    X, Y, Z = (8 * c for c in chunks)
+    nw = np.full((Z, Y, X), 0xFFFFFFFF, np.uint32)
+    for _ in range(3):                                     # chunks of 1..3 request words and empty ones
+        at = rng.random((Z // 8, Y // 8, X // 8)) < 0.4
+        cell = rng.random((8, 8, 8)) < 0.1
+        nw[np.kron(at, np.ones((8, 8, 8), bool)) & np.tile(cell, (Z // 8, Y // 8, X // 8))] = 0x0080FF80
+    vol = Volume(chunks, min_chunks=chunks[0] * chunks[1] * chunks[2])
+    vol.set_material(0)
+    vol.set_dense(nw, np.where(nw == 0xFFFFFFFF, 0, 0x80808000).astype(np.uint32))
+    vol.request_all()
+    vol.sync()
+    o = oracle.load("f32")
+    for _ in range(split):
+        vol.mark_visible(chunks[0] * chunks[1] * chunks[2])
+        before, c, _ = vol.export_state()
+        vol.sync(split=split)
+        req = vol.fetch_requests()
+        assert np.array_equal(req, o.visible_requests(before, c, split=split, frame=int(vol.v.frameNum)))
+        after, _, _ = vol.export_state()
+        assert np.array_equal(after[:, 1], before[:, 1] + 1)
+    assert len(req) > 0
+    vol.close()
