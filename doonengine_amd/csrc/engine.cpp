@@ -15,6 +15,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <exception>
+#include <memory>
+#include <new>
 #include <set>
 #include <thread>
 #include <vector>
@@ -184,6 +186,8 @@ struct DNgpuVolume {
     uint64_t loadedBlocks = 0;
     std::vector<uint32_t> dirty;
     std::vector<uint8_t> dirtyMark;
+    std::unique_ptr<uint4[]> converted;   // stream_chunks: 512 voxels per chunk to load
+    size_t convertedCap = 0;              // in chunks
     bool fullScan = false;
     bool requestAll = false;
     bool resetPending = false;         // a failed upload: clear the device tiles and reload everything
@@ -221,6 +225,8 @@ struct DNgpuVolume {
 };
 
 namespace {
+
+enum { DN_KEEP_CONVERTED = 2048 };   // chunks: 16 MiB
 
 enum { TK_DRAW = 0, TK_LIGHT, TK_VISIBLE, TK_UPLOAD, TK_EPILOGUE, TK_RAYS };
 
@@ -405,30 +411,50 @@ uint32_t chunk_to_gpu(const DNmaterial* mats, const DNchunk& ch, DNchunkRec& rec
 {
     memset(&rec, 0, sizeof(rec));
     rec.pos[0] = ch.pos.x; rec.pos[1] = ch.pos.y; rec.pos[2] = ch.pos.z;
-    auto faceVisible = [&](int x, int y, int z) -> bool {
-        if(x < 0 || y < 0 || z < 0 || x >= 8 || y >= 8 || z >= 8) return true;
-        uint32_t m = material_of(ch.voxels[x][y][z].normal);
-        return m == DN_MATERIAL_EMPTY || mats[m].opacity < 1.0f;
-    };
+    // One bit per cell, x + 8y, a word per z (six tests of neighbours per voxel took most
+    // of an edited frame's conversion): voxels, and cells that show the faces
+    // they touch (empty or see-through)
+    uint64_t solid[8], shows[8];
+    for(int z = 0; z < 8; z++)
+    {
+        uint64_t so = 0, sh = 0;
+        for(int y = 0; y < 8; y++)
+        for(int x = 0; x < 8; x++)
+        {
+            const uint32_t m = material_of(ch.voxels[x][y][z].normal);
+            const uint64_t bit = 1ull << (x + 8 * y);
+            if(m == DN_MATERIAL_EMPTY) sh |= bit;
+            else
+            {
+                so |= bit;
+                if(mats[m].opacity < 1.0f) sh |= bit;
+            }
+        }
+        solid[z] = so;
+        shows[z] = sh;
+    }
+    // a voxel is stored if one of its six neighbours shows its face; cells outside the chunk do
+    const uint64_t X0 = 0x0101010101010101ull, X7 = X0 << 7, Y0 = 0xFFull, Y7 = Y0 << 56, ALL = ~0ull;
     uint32_t n = 0;
     for(int z = 0; z < 8; z++)
-    for(int y = 0; y < 8; y++)
-    for(int x = 0; x < 8; x++)
     {
-        uint32_t index = (uint32_t)(x + 8 * (y + 8 * z));
-        if((index & 127u) == 0 && index != 0) rec.partial[(index >> 7) - 1] = n;
-        const DNcompressedVoxel& v = ch.voxels[x][y][z];
-        if(material_of(v.normal) == DN_MATERIAL_EMPTY) continue;
-        if(!(faceVisible(x + 1, y, z) || faceVisible(x - 1, y, z) || faceVisible(x, y + 1, z) ||
-             faceVisible(x, y - 1, z) || faceVisible(x, y, z + 1) || faceVisible(x, y, z - 1)))
-            continue;
-        rec.mask[index >> 5] |= 1u << (index & 31u);
-        const uint32_t mat = material_of(v.normal);
-        used[mat >> 6] |= 1ull << (mat & 63u);
-        uint32_t a = v.albedo;
-        uint32_t r = g_linLUT[(a >> 24) & 255u], gg = g_linLUT[(a >> 16) & 255u], b = g_linLUT[(a >> 8) & 255u];
-        vox[n] = make_uint4(v.normal, (r << 24) | (gg << 16) | (b << 8), 0u, 0u);
-        n++;
+        const uint64_t s = shows[z];
+        const uint64_t open = ((s >> 1) & ~X7) | X7 | ((s << 1) & ~X0) | X0 | (s >> 8) | Y7 | (s << 8) | Y0 |
+                              (z < 7 ? shows[z + 1] : ALL) | (z > 0 ? shows[z - 1] : ALL);
+        const uint64_t stored = solid[z] & open;
+        if(z == 2 || z == 4 || z == 6) rec.partial[z / 2 - 1] = n;
+        rec.mask[2 * z] = (uint32_t)stored;
+        rec.mask[2 * z + 1] = (uint32_t)(stored >> 32);
+        for(uint64_t left = stored; left; left &= left - 1)
+        {
+            const int i = __builtin_ctzll(left);
+            const DNcompressedVoxel& v = ch.voxels[i & 7][i >> 3][z];
+            const uint32_t mat = material_of(v.normal), a = v.albedo;
+            used[mat >> 6] |= 1ull << (mat & 63u);
+            const uint32_t r = g_linLUT[(a >> 24) & 255u], gg = g_linLUT[(a >> 16) & 255u], b = g_linLUT[(a >> 8) & 255u];
+            vox[n] = make_uint4(v.normal, (r << 24) | (gg << 16) | (b << 8), 0u, 0u);
+            n++;
+        }
     }
     rec.numVoxels = n;
     rec.samples = 0;
@@ -1111,7 +1137,24 @@ void stream_chunks(DNvolume* vol)
 
     // convert the chunks to load (_DN_chunk_to_gpu, on host threads)
     std::vector<DNchunkRec> recs(loads.size());
-    std::vector<uint4> voxBuf(loads.size() * 512);
+    // the volume's buffer of converted voxels, kept up to DN_KEEP_CONVERTED chunks: a new
+    // one each frame costs its clearing and the faults of its pages
+    if(g->convertedCap < loads.size())
+    {
+        g->converted.reset(new (std::nothrow) uint4[loads.size() * 512]);
+        g->convertedCap = g->converted ? loads.size() : 0;
+        if(!g->converted)
+        {
+            dn_msg(DN_MESSAGE_CPU_MEMORY, DN_MESSAGE_ERROR, "chunk streaming postponed: no memory for %zu chunks",
+                   loads.size());
+            return;                              // nothing committed; the dirty tiles stay dirty
+        }
+    }
+    uint4* const voxBuf = g->converted.get();
+    struct Trim {
+        DNgpuVolume* g;
+        ~Trim() { if(g->convertedCap > DN_KEEP_CONVERTED) { g->converted.reset(); g->convertedCap = 0; } }
+    } trim{g};
     std::vector<uint32_t> counts(loads.size());
     if(!loads.empty())
     {
@@ -1128,13 +1171,10 @@ void stream_chunks(DNvolume* vol)
             }
             memcpy(used[w], bits, sizeof(bits));
         };
-        if(nth == 1) work(0);
-        else
-        {
-            std::vector<std::thread> th;
-            for(unsigned w = 0; w < nth; w++) th.emplace_back(work, w);
-            for(auto& x : th) x.join();
-        }
+        std::vector<std::thread> th;
+        for(unsigned w = 1; w < nth; w++) th.emplace_back(work, w);
+        work(0);
+        for(auto& x : th) x.join();
         for(unsigned w = 0; w < nth; w++)
             for(int k = 0; k < 4; k++) g->usedMats[k] |= used[w][k];
     }
